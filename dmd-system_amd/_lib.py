@@ -79,6 +79,9 @@ SIGNATURES = {
                                  _pvp, _pi32, _i32, _pi64, _pi32, _i32, _vp, _i64, _vp]),
     "mlora_f32_seg_outer": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _pvp, _int, _pi32, _i32,
                                    _pi64, _pi32, _i32, _vp]),
+    "mlora_f32_seg_outer_workspace_bytes": (_i64, [_i64, _i64, _pi32, _i32, _pi64, _pi32, _i32]),
+    "mlora_f32_seg_outer_split": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _pvp, _int, _pi32, _i32,
+                                         _pi64, _pi32, _i32, _vp, _i64, _vp]),
 }
 
 _LIB = None

@@ -695,12 +695,16 @@ def f32_seg_outer(p: torch.Tensor, h: torch.Tensor, ranks: Sequence[int], routin
     shape = (lambda r: (C, r)) if out_layout == 0 else (lambda r: (r, C))
     outs: list[torch.Tensor | None] = [None] * len(ranks)
     stream = _stream(p)
+    rk = _lib.i32_array(list(ranks))
     for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
         o, i, n = _routing_arrays(off, ids)
-        part = [torch.zeros(shape(r), dtype=torch.float32, device=p.device) for r in ranks]
-        _lib.check("mlora_f32_seg_outer", lib.mlora_f32_seg_outer(
+        part = [torch.empty(shape(r), dtype=torch.float32, device=p.device) for r in ranks]
+        ws_bytes = lib.mlora_f32_seg_outer_workspace_bytes(r1 - r0, C, rk, len(ranks), o, i, n)
+        _lib.check("mlora_f32_seg_outer_workspace_bytes", ws_bytes if ws_bytes < 0 else 0)
+        ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=p.device) if ws_bytes else None
+        _lib.check("mlora_f32_seg_outer_split", lib.mlora_f32_seg_outer_split(
             p[r0:r1].data_ptr(), p.stride(0), r1 - r0, C, h[r0:r1].data_ptr(), h.stride(0),
-            _lib.ptr_array([t.data_ptr() for t in part]), out_layout, _lib.i32_array(list(ranks)), len(ranks),
-            o, i, n, stream))
+            _lib.ptr_array([t.data_ptr() for t in part]), out_layout, rk, len(ranks), o, i, n, _ptr(ws), ws_bytes,
+            stream))
         outs = [t if acc is None else acc + t for acc, t in zip(outs, part)]
     return outs  # type: ignore[return-value]

@@ -448,6 +448,20 @@ int mlora_f32_seg_outer(const void *p, int64_t ldp, int64_t M, int64_t C,
                         const int64_t *seg_offsets, const int32_t *adapter_ids, int32_t n_segments,
                         void *stream);
 
+/* The same with every adapter's rows split over several workgroups: partial sums in
+ * `workspace` (16-byte aligned, at least mlora_f32_seg_outer_workspace_bytes of the same
+ * arguments; 0 bytes: may be NULL), added in split order (deterministic). */
+int64_t mlora_f32_seg_outer_workspace_bytes(int64_t M, int64_t C, const int32_t *ranks, int32_t n_adapters,
+                                            const int64_t *seg_offsets, const int32_t *adapter_ids,
+                                            int32_t n_segments);
+int mlora_f32_seg_outer_split(const void *p, int64_t ldp, int64_t M, int64_t C,
+                              const void *h, int64_t ldh,
+                              void *const *out_ptrs, int out_layout,
+                              const int32_t *ranks, int32_t n_adapters,
+                              const int64_t *seg_offsets, const int32_t *adapter_ids, int32_t n_segments,
+                              void *workspace, int64_t workspace_bytes,
+                              void *stream);
+
 #ifdef __cplusplus
 }
 #endif
