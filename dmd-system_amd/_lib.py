@@ -58,6 +58,10 @@ SIGNATURES = {
     "mlora_modulated_norm_component_grad": (_int, [_vp, _int, _i64, _i64, _vp, _int, _i64, _i64, _vp, _vp,
                                                    _vp, _int, _i64, _i64, _i64, _int, _int, _int, _vp, _i64,
                                                    _i64, _i64, _i64, _vp]),
+    "mlora_modulated_norm_backward_fused_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "mlora_modulated_norm_backward_fused": (_int, [_vp, _int, _i64, _i64, _vp, _int, _i64, _i64, _vp, _int,
+                                                   _vp, _int, _i64, _vp, _i64, _i64, ctypes.c_float, _int, _int,
+                                                   _vp, _int, _vp, _int, _vp, _i64, _i64, _i64, _i64, _vp]),
     "mlora_gemm_dx": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _i64,
                              _pvp, _pi32, _i32, _pi64, _pi32, _i32, _vp, _i64, _int, _vp]),
     "mlora_seg_outer": (_int, [_vp, _i64, _i64, _i64, _vp, _i32, _pvp, _int, _int, _pi32, _i32,

@@ -35,6 +35,8 @@
 #include "mlora_common.h"
 #include "mlora_host.h"
 
+#include <type_traits>
+
 namespace mlora {
 
 constexpr int kNormMaxWidth = 8192;
@@ -463,6 +465,215 @@ __global__ __launch_bounds__(64 * kNormRowsPerBlock) void norm_component_token_k
   }
 }
 
+// Fused backward of the broadcast modulation (scale constant over a sample's tokens): dx and the
+// component sums Σ_t g·n, Σ_t g in one pass over x and g. HBM-bound: the sums used to be a second
+// pass over both.
+//
+// A workgroup takes `chunk` consecutive tokens of one sample and leaves one partial sum. A row
+// belongs to WPR of its 4 waves (their row sums meet in LDS, added in wave order), NCH chunks of 8
+// features per lane, so that the row, its gradient, the hoisted RN(1 + s) and the two running
+// sums stay in registers (at most 194, two waves per SIMD; capping them at 128 or 168 spills and
+// measured 1.7-2.5x slower): one wave holds rows up to 1536 features, two up to 3072, four up to
+// 5120. The 4 / WPR row streams of the workgroup are added in stream order.
+// At 65520 x 1536, float32 stream: 212 us for dx and the sums (4.8 TB/s of the 1.01 GB it must
+// move) against 193 + 129 us for the two passes.
+struct NormBwdFusedArgs {
+  NormBwdArgs b;
+  float *partial;  // [batches, n_chunks, 2, width]
+  int32_t n_chunks, chunk;
+};
+
+template <int NCH, int WPR, bool XF32, bool GF32>
+__global__ __launch_bounds__(64 * kNormRowsPerBlock) void norm_backward_fused_kernel(const NormBwdFusedArgs fa) {
+  const NormBwdArgs &a = fa.b;
+  constexpr int NW = kNormRowsPerBlock, STREAMS = NW / WPR;
+  __shared__ float red[WPR > 1 ? 4 * NW : 1];
+  __shared__ f32x4 sums[NCH * WPR * 64 * 4];  // one row of Σ g·n, then of Σ g (8 features = 2 vectors each)
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int sub = wave % WPR, stream = wave / WPR;
+  const int nchunks = a.width / 8;
+  const float width = (float)a.width;
+  const int64_t b = blockIdx.x / fa.n_chunks;
+  const int tc = blockIdx.x % fa.n_chunks;
+  const int t0 = tc * fa.chunk, t1 = min(t0 + fa.chunk, a.tokens);
+  // a row's sum over the waves that hold it, in wave order (slot: one per use between barriers)
+  auto row_sum = [&](float v, int slot) -> float {
+    v = wave_sum(v);
+    if constexpr (WPR == 1) return v;
+    if (lane == 0) red[slot * NW + wave] = v;
+    __syncthreads();
+    float s = red[slot * NW + stream * WPR];
+#pragma unroll
+    for (int w = 1; w < WPR; ++w) s += red[slot * NW + stream * WPR + w];
+    return s;
+  };
+  float ops[NCH][8], sgn[NCH][8], sg[NCH][8];  // RN(1 + s); Σ g·n; Σ g
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    const int c = lane + 64 * (k * WPR + sub);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ops[k][i] = 0.f, sgn[k][i] = 0.f, sg[k][i] = 0.f;
+    if (c < nchunks) {
+      load8(a.scale, a.scale_f32, b * a.scale_sb + 8 * c, ops[k]);
+      if (a.scale_row != nullptr) {
+        float ts[8];
+        load8(a.scale_row, a.table_f32, 8 * c, ts);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ops[k][i] = add_rn(ts[i], ops[k][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ops[k][i] = add_rn(1.0f, ops[k][i]);
+    }
+  }
+  // every stream runs the same number of rows, so that every wave meets the same barriers; a
+  // stream past the chunk's end reads and writes nothing
+  for (int t = t0 + stream; t - stream < t1; t += STREAMS) {
+    const bool live = t < t1;
+    float x[NCH][8], g[NCH][8];
+    const int64_t xo = b * a.x_sb + t * a.x_st, go = b * a.g_sb + t * a.g_st;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const int c = lane + 64 * (k * WPR + sub);
+      if (live && c < nchunks) {
+        load8(a.x, XF32, xo + 8 * c, x[k]);
+        load8(a.g, GF32, go + 8 * c, g[k]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[k][i] = 0.f, g[k][i] = 0.f;
+      }
+    }
+    float s1 = 0.f;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s1 += x[k][i];
+    const float mean = row_sum(s1, 0) / width;
+    float s2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const bool in = lane + 64 * (k * WPR + sub) < nchunks;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float c = x[k][i] - mean;
+        x[k][i] = c;
+        if (in) s2 += c * c;
+      }
+    }
+    const float rstd = 1.0f / __fsqrt_rn(row_sum(s2, 1) / width + a.eps);
+    // x -> n; the component sums; gn = RN(g · RN(1 + s)) into g; the two row sums
+    float rg = 0.f, rgn = 0.f;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const bool in = live && lane + 64 * (k * WPR + sub) < nchunks;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[k][i] = mul_rn(x[k][i], rstd);
+        if (in) {
+          sgn[k][i] += g[k][i] * x[k][i];
+          sg[k][i] += g[k][i];
+        }
+        g[k][i] = mul_rn(g[k][i], ops[k][i]);
+        if (in) {
+          rg += g[k][i];
+          rgn += g[k][i] * x[k][i];
+        }
+      }
+    }
+    const float gsum_w = row_sum(rg, 2) / width, gnn_w = row_sum(rgn, 3) / width;
+    const int64_t dxo = b * a.dx_sb + t * a.dx_st;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const int c = lane + 64 * (k * WPR + sub);
+      if (!live || c >= nchunks) continue;
+      float d[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d[i] = ln_input_grad(g[k][i], x[k][i], gsum_w, gnn_w, rstd);
+      store8_any(a.dx, XF32, dxo + 8 * c, d);
+    }
+  }
+  // the streams' sums, added in stream order through LDS
+  constexpr int ROW = NCH * WPR * 64 * 2;  // vectors of one sum
+#pragma unroll
+  for (int w = 0; w < STREAMS; ++w) {
+    if (stream == w) {
+#pragma unroll
+      for (int k = 0; k < NCH; ++k) {
+        const int c = lane + 64 * (k * WPR + sub);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float *src = q < 2 ? &sgn[k][4 * q] : &sg[k][4 * (q - 2)];
+          f32x4 v = f32x4{src[0], src[1], src[2], src[3]};
+          f32x4 &dst = sums[(q >> 1) * ROW + 2 * c + (q & 1)];
+          if (w > 0) v += dst;
+          dst = v;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  float *p = fa.partial + ((int64_t)b * fa.n_chunks + tc) * 2 * a.width;
+  for (int v = threadIdx.x; v < 4 * nchunks; v += 64 * NW) {
+    const int k = v / (2 * nchunks), e = v % (2 * nchunks);
+    *(MLORA_GLOBAL f32x4 *)(p + k * a.width + 4 * e) = sums[k * ROW + e];
+  }
+}
+
+// The component gradient [batches, 6, width] (zeros in the other four slots) and its sum over the
+// samples, the table gradient [6, width], from the partial sums: one wave per (slot, 8-feature
+// chunk), lane l adding chunks l, l + 64, ... of a sample in order, then a butterfly.
+struct NormCompFinishArgs {
+  const float *partial;
+  void *d_comp, *d_table;  // either may be null
+  int32_t batches, width, n_chunks, si, hi, comp_f32, table_f32;
+};
+
+__global__ __launch_bounds__(64 * kNormRowsPerBlock) void norm_component_finish_kernel(const NormCompFinishArgs a) {
+  const int lane = threadIdx.x & 63, nchunks = a.width / 8;
+  const int wv = blockIdx.x * kNormRowsPerBlock + wave_id();
+  if (wv >= 6 * nchunks) return;
+  const int slot = wv / nchunks, c = wv % nchunks;
+  const bool live = slot == a.si || slot == a.hi;
+  const int64_t per = 2 * (int64_t)a.width;
+  float table = 0.f;  // lane i < 8: feature 8c + i
+  auto store = [&](void *base, bool f32, int64_t e, float v) {
+    if (f32) static_cast<float *>(base)[e] = v;
+    else static_cast<uint16_t *>(base)[e] = f32_to_bf16_rne(v);
+  };
+  for (int b = 0; b < a.batches; ++b) {
+    float mine = 0.f;
+    if (live) {
+      const float *p = a.partial + (int64_t)b * a.n_chunks * per + (slot == a.si ? 0 : a.width) + 8 * c;
+      float acc[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+      for (int tc = lane; tc < a.n_chunks; tc += 64) {
+        float v[8];
+        load8(p + (int64_t)tc * per, true, 0, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] += v[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float v = wave_sum(acc[i]);
+        mine = lane == i ? v : mine;
+      }
+    }
+    table += mine;
+    if (lane < 8 && a.d_comp != nullptr) store(a.d_comp, a.comp_f32, ((int64_t)b * 6 + slot) * a.width + 8 * c + lane, mine);
+  }
+  if (lane < 8 && a.d_table != nullptr) store(a.d_table, a.table_f32, (int64_t)slot * a.width + 8 * c + lane, table);
+}
+
+// Tokens per workgroup: the fewest (a power of two, 8 to 128) that leave at most 512 workgroups, the
+// number that run at once (two waves per SIMD). With the finishing kernel, float32 stream: 65520 x
+// 1536 220 us at 128 tokens, 227 at 64, 235 at 32; 32760 x 3072 220 at 64, 227 at 32; 16380 x 5120
+// 193 at 32, 209 at 16, 289 at 64; 4680 x 1536 28 at 16, 33 at 8, 35 at 32.
+static int fused_chunk(int64_t batches, int64_t tokens) {
+  int chunk = 8;
+  while (chunk < 128 && batches * ((tokens + chunk - 1) / chunk) > 512) chunk *= 2;
+  return chunk;
+}
+
 // Rows of 16-byte chunks: every row start 16-byte aligned.
 static bool rows_aligned(const void *p, int64_t sb, int64_t st) {
   return aligned16(p) && sb >= 0 && st >= 0 && sb % 8 == 0 && st % 8 == 0;
@@ -616,5 +827,77 @@ extern "C" int mlora_modulated_norm_component_grad(const void *x, int x_dtype, i
   const int64_t rows = batches * tokens;
   hipLaunchKernelGGL(norm_component_token_kernel, dim3((unsigned)((rows + kNormRowsPerBlock - 1) / kNormRowsPerBlock)),
                      dim3(64 * kNormRowsPerBlock), 0, s, a);
+  return launch_status();
+}
+
+extern "C" int64_t mlora_modulated_norm_backward_fused_workspace_bytes(int64_t batches, int64_t tokens, int64_t width) {
+  if (batches < 0 || tokens < 0 || width < 0) return MLORA_ERR_INVALID;
+  if (batches == 0 || tokens == 0) return 0;
+  if (tokens > INT32_MAX / batches) return MLORA_ERR_LIMIT;
+  const int64_t chunk = fused_chunk(batches, tokens);
+  return batches * ((tokens + chunk - 1) / chunk) * 2 * width * (int64_t)sizeof(float);
+}
+
+extern "C" int mlora_modulated_norm_backward_fused(const void *x, int x_dtype, int64_t x_sb, int64_t x_st,
+                                                   const void *g, int g_dtype, int64_t g_sb, int64_t g_st,
+                                                   const void *scale_row, int table_dtype,
+                                                   const void *scale, int scale_dtype, int64_t scale_sb,
+                                                   void *dx, int64_t dx_sb, int64_t dx_st, float eps,
+                                                   int scale_index, int shift_index, void *d_comp, int d_comp_dtype,
+                                                   void *d_table, int d_table_dtype, void *workspace,
+                                                   int64_t workspace_bytes, int64_t batches, int64_t tokens,
+                                                   int64_t width, void *stream) {
+  if (batches < 0 || tokens < 0 || width < 0) return MLORA_ERR_INVALID;
+  for (int d : {x_dtype, g_dtype, scale_dtype, d_comp_dtype, d_table_dtype})
+    if (d != MLORA_BF16 && d != MLORA_F32) return MLORA_ERR_UNSUPPORTED;
+  if (scale_row != nullptr && table_dtype != MLORA_BF16 && table_dtype != MLORA_F32) return MLORA_ERR_UNSUPPORTED;
+  if (!(eps > 0.f && eps < INFINITY)) return MLORA_ERR_INVALID;
+  if (scale_index < 0 || scale_index >= 6 || shift_index < 0 || shift_index >= 6 || scale_index == shift_index)
+    return MLORA_ERR_INVALID;
+  if (width > 0 && (width % 8 != 0 || width > kNormBwdMaxWidth)) return MLORA_ERR_UNSUPPORTED;
+  if (batches > 0 && tokens > INT32_MAX / batches) return MLORA_ERR_LIMIT;
+  const int64_t rows = batches * tokens;
+  if (rows > INT32_MAX - kNormRowsPerBlock) return MLORA_ERR_LIMIT;
+  if (rows == 0 || width == 0) return MLORA_OK;
+  if (x == nullptr || g == nullptr || scale == nullptr || dx == nullptr) return MLORA_ERR_INVALID;
+  if (tokens > 1 && dx_st < width) return MLORA_ERR_INVALID;  // rows of one batch overlap
+  if (batches > 1 && dx_sb < (tokens - 1) * dx_st + width) return MLORA_ERR_INVALID;  // batches overlap
+  if (!rows_aligned(x, x_sb, x_st) || !rows_aligned(g, g_sb, g_st) || !rows_aligned(scale, scale_sb, 0) ||
+      !rows_aligned(dx, dx_sb, dx_st))
+    return MLORA_ERR_UNSUPPORTED;
+  if (scale_row != nullptr && !aligned16(scale_row)) return MLORA_ERR_UNSUPPORTED;
+  const int64_t need = mlora_modulated_norm_backward_fused_workspace_bytes(batches, tokens, width);
+  if (workspace == nullptr || workspace_bytes < need) return MLORA_ERR_WORKSPACE;
+  if (!aligned16(workspace)) return MLORA_ERR_UNSUPPORTED;
+  const int chunk = fused_chunk(batches, tokens);
+  NormBwdFusedArgs a{{x, g, scale_row, scale, dx, nullptr, nullptr, x_sb, x_st, g_sb, g_st, scale_sb, 0, dx_sb, dx_st,
+                      (int32_t)rows, (int32_t)tokens, (int32_t)width, x_dtype == MLORA_F32, g_dtype == MLORA_F32,
+                      table_dtype == MLORA_F32, scale_dtype == MLORA_F32, x_dtype == MLORA_F32, eps},
+                     static_cast<float *>(workspace), (int32_t)((tokens + chunk - 1) / chunk), chunk};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)(batches * a.n_chunks)), block(64 * kNormRowsPerBlock);
+  const int n = (int)((width / 8 + 63) / 64);  // chunks of 8 features per lane of one wave
+  auto launch = [&](auto nch, auto wpr) {
+    constexpr int NCH = decltype(nch)::value, WPR = decltype(wpr)::value;
+    const bool xf = x_dtype == MLORA_F32, gf = g_dtype == MLORA_F32;
+    if (xf && gf) hipLaunchKernelGGL((norm_backward_fused_kernel<NCH, WPR, true, true>), grid, block, 0, s, a);
+    else if (xf) hipLaunchKernelGGL((norm_backward_fused_kernel<NCH, WPR, true, false>), grid, block, 0, s, a);
+    else if (gf) hipLaunchKernelGGL((norm_backward_fused_kernel<NCH, WPR, false, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((norm_backward_fused_kernel<NCH, WPR, false, false>), grid, block, 0, s, a);
+  };
+  using std::integral_constant;
+  if (n <= 1) launch(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  else if (n <= 2) launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else if (n <= 3) launch(integral_constant<int, 3>{}, integral_constant<int, 1>{});
+  else if (n <= 4) launch(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+  else if (n <= 6) launch(integral_constant<int, 3>{}, integral_constant<int, 2>{});
+  else if (n <= 8) launch(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+  else launch(integral_constant<int, 3>{}, integral_constant<int, 4>{});
+  int st = launch_status();
+  if (st || (d_comp == nullptr && d_table == nullptr)) return st;
+  const NormCompFinishArgs f{a.partial, d_comp, d_table, (int32_t)batches, (int32_t)width, a.n_chunks, scale_index,
+                             shift_index, d_comp_dtype == MLORA_F32, d_table_dtype == MLORA_F32};
+  const int waves = 6 * (int)(width / 8);
+  hipLaunchKernelGGL(norm_component_finish_kernel, dim3((waves + kNormRowsPerBlock - 1) / kNormRowsPerBlock), block, 0, s, f);
   return launch_status();
 }

@@ -394,6 +394,38 @@ def modulated_norm_component_grad(x: torch.Tensor, g: torch.Tensor, mean: torch.
     return out
 
 
+def modulated_norm_backward_fused(x: torch.Tensor, g: torch.Tensor, scale: torch.Tensor, scale_row: torch.Tensor,
+                                  dx: torch.Tensor, d_comp: torch.Tensor | None, d_table: torch.Tensor | None, *,
+                                  scale_index: int, shift_index: int, eps: float) -> torch.Tensor:
+    """modulated_norm_backward for a scale [B, W] constant over a sample's tokens, with the component
+    gradient in the same pass: d_comp [B, 6, W] (Σ_t g·n, Σ_t g, zeros in the other slots) and
+    d_table [1, 6, W] (d_comp summed over the samples), contiguous, either None."""
+    B, T, W = x.shape
+    fl = (torch.bfloat16, torch.float32)
+    _rows3("hidden", x, fl, (B, T, W))
+    _rows3("grad_output", g, fl, (B, T, W))
+    _rows3("hidden_gradient", dx, (x.dtype,), (B, T, W))
+    for name, t, shape in (("scale_component", scale, (B, W)), ("scale_row", scale_row, (W,)),
+                           ("component gradient", d_comp, (B, 6, W)), ("table gradient", d_table, (1, 6, W))):
+        _require(t is None or (t.is_cuda and t.dtype in fl and tuple(t.shape) == shape and t.stride(-1) == 1),
+                 f"{name} must be a {list(shape)} bfloat16 or float32 device tensor with unit feature stride")
+    for name, t in (("component gradient", d_comp), ("table gradient", d_table)):
+        _require(t is None or t.is_contiguous(), f"{name} must be contiguous")
+    _require(eps > 0, "LayerNorm epsilon must be positive")
+    lib = _lib.load()
+    nbytes = lib.mlora_modulated_norm_backward_fused_workspace_bytes(B, T, W)
+    _lib.check("mlora_modulated_norm_backward_fused_workspace_bytes", nbytes if nbytes < 0 else 0)
+    ws = torch.empty(max(nbytes, 16) // 4, dtype=torch.float32, device=x.device)
+    _lib.check("mlora_modulated_norm_backward_fused", lib.mlora_modulated_norm_backward_fused(
+        x.data_ptr(), _DT[x.dtype], x.stride(0), x.stride(1), g.data_ptr(), _DT[g.dtype], g.stride(0), g.stride(1),
+        scale_row.data_ptr(), _DT[scale_row.dtype], scale.data_ptr(), _DT[scale.dtype], scale.stride(0),
+        dx.data_ptr(), dx.stride(0), dx.stride(1), float(eps), int(scale_index), int(shift_index),
+        _ptr(d_comp), _DT[d_comp.dtype] if d_comp is not None else _lib.F32,
+        _ptr(d_table), _DT[d_table.dtype] if d_table is not None else _lib.F32, ws.data_ptr(), ws.numel() * 4,
+        B, T, W, _stream(x)))
+    return dx
+
+
 def gemm_dx(dy: torch.Tensor, w: torch.Tensor, g_rows: torch.Tensor | None, as_: Sequence[torch.Tensor],
             routing: SegmentRouting, out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
     """dX = dY·W + per-segment g_rows·A_a, bf16 out (accumulate: dX += ..., into `out`).

@@ -259,6 +259,16 @@ class ModulatedLayerNormFunction(torch.autograd.Function):
         si, hi = ctx.idx
         B, T, W = hidden.shape
         g = grad_out.contiguous()
+        if component.dim() == 3 and hidden.numel() and (ctx.needs_input_grad[1] or ctx.needs_input_grad[2]):
+            # one modulation per sample: dx and the component sums in one pass over hidden and g
+            dx = torch.empty_like(hidden)
+            d_comp = (torch.empty(component.shape, dtype=component.dtype, device=hidden.device)
+                      if ctx.needs_input_grad[2] else None)
+            d_table = (torch.empty(table.shape, dtype=table.dtype, device=hidden.device)
+                       if ctx.needs_input_grad[1] else None)
+            kernels.modulated_norm_backward_fused(hidden, g, component[:, si], table[0, si], dx, d_comp, d_table,
+                                                  scale_index=si, shift_index=hi, eps=ctx.eps)
+            return dx, d_table, d_comp, None, None, None
         scale_c = (component[:, si].unsqueeze(1).expand(B, T, W) if component.dim() == 3
                    else component[:, :, si])
         dx = torch.empty_like(hidden)

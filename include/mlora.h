@@ -281,6 +281,24 @@ int mlora_modulated_norm_component_grad(const void *x, int x_dtype, int64_t x_st
                                         int64_t batches, int64_t tokens, int64_t width,
                                         void *stream);
 
+/* dx and the reduced component gradient in one pass, for a scale that is constant over a sample's
+ * tokens (scale [batches, width], batch stride scale_stride_b): dx as mlora_modulated_norm_backward
+ * (in x's dtype), d_comp [batches, 6, width] as reduce 1 above with zeros in the other four slots,
+ * d_table [6, width] = Σ_b d_comp (both contiguous, either may be NULL). Partial sums in a caller
+ * workspace of mlora_modulated_norm_backward_fused_workspace_bytes bytes (16-byte aligned), added in
+ * a fixed order. */
+int64_t mlora_modulated_norm_backward_fused_workspace_bytes(int64_t batches, int64_t tokens, int64_t width);
+int mlora_modulated_norm_backward_fused(const void *x, int x_dtype, int64_t x_stride_b, int64_t x_stride_t,
+                                        const void *g, int g_dtype, int64_t g_stride_b, int64_t g_stride_t,
+                                        const void *scale_row, int table_dtype,
+                                        const void *scale, int scale_dtype, int64_t scale_stride_b,
+                                        void *dx, int64_t dx_stride_b, int64_t dx_stride_t, float eps,
+                                        int scale_index, int shift_index,
+                                        void *d_comp, int d_comp_dtype, void *d_table, int d_table_dtype,
+                                        void *workspace, int64_t workspace_bytes,
+                                        int64_t batches, int64_t tokens, int64_t width,
+                                        void *stream);
+
 /* Input gradient with the LoRA term fused into its epilogue:
  *   dX[m, k] = bf16( Σ_n dY[m,n]·W[n,k] + Σ_j g_rows[m,j]·A_a[j,k] )
  * g_rows = s_a·dY·B_a from mlora_shrink(op_layout=1). a_ptrs[i]: bf16 [r_i, K].
