@@ -72,7 +72,7 @@ struct GemmArgs {
 };
 
 template <int BM_, int BN_, int WM_, int WN_, bool NN_, bool F8_ = false, int KB_ = 128, int STAGES_ = 2,
-          bool RING5_ = false, bool SPREAD_ = false, bool PP_ = false>
+          bool RING5_ = false, bool SPREAD_ = false, bool PP_ = false, bool RB_ = false>
 struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr bool NN = NN_;
@@ -127,6 +127,10 @@ struct GemmCfg {
   // PP: the ping-pong schedule of contract_tile_pp (8-wave 256x256 bf16 NT tiles; its own LDS ring)
   static constexpr bool PP = PP_;
   static_assert(!PP || (RING5 && !F8 && !NN && NW == 8), "the ping-pong schedule runs 8-wave bf16 NT tiles on the 5-slot ring");
+  // RB: a whole k-tile of fragments in registers, the next one's read during a step's MFMAs
+  // (small bf16 NT tiles: see contract_tile)
+  static constexpr bool RB = RB_;
+  static_assert(!RB || (!RING5 && !F8 && !NN && STAGES >= 2), "register-buffered steps: bf16 NT tiles in plain stages");
   static constexpr int p_off(int ph) { return RING5 ? ((2 * ph) % 5) * A_BYTES : ph * A_BYTES; }
   static constexpr int q_off(int ph) { return RING5 ? ((2 * ph + 1) % 5) * A_BYTES : ph * B_BYTES; }
   static_assert(LDS_BYTES <= 163840, "the ring must fit the 160 KB of LDS");
@@ -216,6 +220,19 @@ struct Pipe {
       }
       b_kc[0] = b_kc[1] = rl;  // row of this lane within its 1 KB load
     }
+  }
+
+  // Load number Q of a k-tile that needs no mask (whole, every P row of this source; NT).
+  template <int Q>
+  __device__ __forceinline__ void issue_whole(MLORA_LDS char *lds, int ph, int k0, int wave) const {
+    constexpr bool IS_P = Q < C::A_DMA;
+    constexpr int q = IS_P ? Q : Q - C::A_DMA, D = IS_P ? C::A_DMA : C::B_DMA;
+    const int blk = wave * D + q;
+    MLORA_LDS void *dst = lds + (IS_P ? C::p_off(ph) : C::B_BASE + C::q_off(ph)) + blk * 1024;
+    const int32_t(&o)[2] = IS_P ? a_off : b_off;
+    const int32_t off = (D % 2 == 0 ? q % 2 : blk % 2) ? o[1] : o[0];
+    const int32_t soff = C::RPD * blk * (IS_P ? ldp_b : ldq_b) + k0 * 2;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(IS_P ? rp : rq, dst, 16, off, soff, 0, 0);
   }
 
   // Issue 1 KB load number q (of NDMA per wave) of the k-tile starting at k0
@@ -607,6 +624,57 @@ __device__ __forceinline__ void contract_tile(f32x16 (&acc)[C::TM][C::TN], const
   // barrier)
   constexpr int PQ = C::RING5 ? C::A_DMA : 0;  // loads of a step issued before its barrier
   constexpr int WAIT = C::RING5 ? PQ : (C::AHEAD - 2) * NDMA;
+  if constexpr (C::RB) {
+    // Register-buffered steps: step t multiplies k-tile t from registers while every fragment of
+    // k-tile t+1 is read from LDS and the loads of k-tile t+S go to the stage of k-tile t, whose
+    // fragments were all read in the step before. A small tile's substep is one or two MFMAs
+    // (32 cycles each), less than an LDS read takes, so reading substep by substep made a step four
+    // LDS latencies long; this one waits for one. Same MFMA order: the same result bit for bit.
+    constexpr int UN = S % 2 == 0 ? S : 2 * S;  // steps until stages and register buffers repeat
+    constexpr int NM = NSUB * C::TMN;
+    Half<C> f0[NSUB], f1[NSUB];
+    static_for<NSUB>([&](auto h) {
+      read_half<C, 0>(f0[decltype(h)::value], decltype(h)::value, lds, fa);
+      return true;
+    });
+    // k-tiles of the current source that are whole and, for P, of rows of this segment only: their
+    // loads need no masks (the walk and the mask decisions took longer than a small tile's MFMAs)
+    int whole = pipe.p_rows > 0 ? 0 : pipe.klim / bk;
+    while (!done) static_for<UN>([&](auto u) -> bool {
+        constexpr int U = decltype(u)::value, ST = U % S, NS = (U + 1) % S;
+        Half<C>(&x)[NSUB] = U % 2 == 0 ? f0 : f1;
+        Half<C>(&y)[NSUB] = U % 2 == 0 ? f1 : f0;
+        wait_vmcnt<WAIT>();  // this wave's loads of k-tile t + 1
+        lds_pipeline_barrier();
+        static_for<NSUB>([&](auto h) {
+          read_half<C, NS>(y[decltype(h)::value], decltype(h)::value, lds, fa);
+          return true;
+        });
+        if (t_in_src + 1 < whole) {  // k-tile t + S
+          ++t_in_src;
+          ++n_real;
+          static_for<NDMA>([&](auto q) {
+            pipe.template issue_whole<decltype(q)::value>(lds, ST, t_in_src * bk, wave);
+            return true;
+          });
+        } else {
+          const bool live = advance();
+          whole = pipe.p_rows > 0 ? 0 : pipe.klim / bk;
+#pragma unroll
+          for (int q = 0; q < NDMA; ++q) pipe.issue_one(lds, q, ST, t_in_src * bk, wave, lane, kmask, live);
+        }
+#pragma unroll
+        for (int g = 0; g < NM; ++g) {
+          const int h = g / C::TMN, j = g % C::TMN / C::TM, i = g % C::TM;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(x[h].b[j]), as_bf16x8(x[h].a[i]), acc[i][j], 0, 0, 0);
+        }
+        ++t;
+        done = t >= n_real;
+        return !done;
+      });
+    wait_vmcnt<0>();
+    return;
+  }
   Half<C> h0, h1;  // fragments of the current and the next substep
   if constexpr (C::F8) {
     // e4m3 steps (NSUB / 2 substeps of TMN scaled MFMAs), the same barrier
@@ -1293,13 +1361,20 @@ using CfgNT256 = GemmCfg<256, 256, 4, 2, false, false, 128, 2, true, true, true>
 using CfgF8256 = GemmCfg<256, 256, 4, 2, false, true, 128, 2, true, true>;
 using CfgF8128 = GemmCfg<128, 128, 2, 2, false, true>;
 using CfgNN256 = GemmCfg<256, 256, 4, 2, true, false, 128, 2, true, true>;
-using CfgNT128 = GemmCfg<128, 128, 2, 2, false>;
 using CfgNN128 = GemmCfg<128, 128, 2, 2, true>;
-// 128x128 tiles of 8 waves (32x64 each) with three stages (two k-tiles in flight), one workgroup
+// NT grids of fewer than 256 tiles of 256x256 (dispatch_nt). Register-buffered steps where a substep
+// is one or two MFMAs: 64x64 tiles of 4 waves (32x32 each; 48 KB, three workgroups per CU) and 128x128
+// tiles of 8 waves (64x32 each; 96 KB), also the quarters of a partly filled last round of 256x256
+// tiles. 128x256 and 256x128 tiles of 8 waves (64x64 each), three stages.
+using CfgNT64 = GemmCfg<64, 64, 2, 2, false, false, 128, 3, false, false, false, true>;
+using CfgNT128 = GemmCfg<128, 128, 2, 4, false, false, 128, 3, false, false, false, true>;
+using CfgNT128x256 = GemmCfg<128, 256, 2, 4, false, false, 128, 3>;
+using CfgNT256x128 = GemmCfg<256, 128, 4, 2, false, false, 128, 3>;
+// 128x128 NN tiles of 8 waves (64x32 each) with three stages (two k-tiles in flight), one workgroup
 // per CU: grids of at most 256 such tiles, and the quarters of a partly filled last round of
-// 256x256 tiles (dispatch_gemm)
-using CfgNT128W = GemmCfg<128, 128, 4, 2, false, false, 128, 3>;
-using CfgNN128W = GemmCfg<128, 128, 4, 2, true, false, 128, 3>;
+// 256x256 tiles (dispatch_nn)
+using CfgNN128W = GemmCfg<128, 128, 2, 4, true, false, 128, 3>;
+using CfgF864 = GemmCfg<64, 64, 2, 2, false, true, 128, 3>;
 
 // Row tiles per group of the tile order: an XCD's 32 concurrent 256x256 tiles
 // then cover 4 row tiles x up to 8 column tiles (P, streamed from HBM, shared
@@ -1335,14 +1410,6 @@ static int launch_tail(GemmArgs &a, hipStream_t stream, int64_t first) {
   return launch_status();
 }
 
-// Tile choice (measured on MI355X):
-// * At least 256 tiles of 256x256: the 8-wave 256x256 tile (the persistent form whose k-tile ring
-//   runs across output tiles, and 256x128 tiles with a 3-stage ring, both measured slower).
-// * Fewer, and at most 256 tiles of 128x128: one 8-wave 128x128 workgroup per CU with three
-//   stages (CfgNT128W / CfgNN128W), 15-35% faster than the 4-wave two-stage tile, two per CU, at
-//   48-192 tiles (512-2048 rows, K 1536-8960); with more tiles (two rounds or more of one
-//   workgroup per CU) it measured 2-32% slower (7% faster only for a forward at K = 3072).
-// * Otherwise the 4-wave two-stage 128x128 tile, two workgroups per CU.
 // A grid of 256x256 tiles a little over whole rounds of the 256 CUs (1284 tiles at 27280 x 3072:
 // five rounds and four tiles) would spend a whole tile's time on its last few tiles. Those
 // tiles (at most 64, the last of the tile order) then run in a second launch as 128x128
@@ -1350,30 +1417,75 @@ static int launch_tail(GemmArgs &a, hipStream_t stream, int64_t first) {
 // 27280 x 3072 forward and NN dX took 10% and 7% less time per launch, its step 2.9% less.
 // (The 4-wave two-stage 128x128 tile was no faster than no split. Tails of 104 and 128 tiles,
 // two rounds of quarters, were 2-6% faster per launch in isolation but left config 4's step
-// 0.6% slower.) Every output keeps the same k order and MFMA sequence in all tile sizes, so
-// the result is the same bit for bit. The e4m3 GEMM keeps the 4-wave 128x128 tile for small
-// grids and its tail as 256x256 tiles (its 8-wave quarters measured 1% slower).
-template <class Big, class Small, bool RESID = false, int STK = 0>
-static int dispatch_gemm(GemmArgs &a, hipStream_t stream) {
-  constexpr int64_t kCUs = 256, kMaxTail = 64;
-  using Wide = std::conditional_t<Big::F8, void, std::conditional_t<Big::NN, CfgNN128W, CfgNT128W>>;
-  const int64_t big_tiles = (int64_t)((a.M + 255) / 256) * ((a.Ncols + 255) / 256);
-  if (big_tiles < kCUs) {
-    if constexpr (!std::is_void_v<Wide>) {
-      const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.Ncols + 127) / 128);
-      if (tiles <= kCUs) return launch_gemm<Wide, RESID, STK>(a, stream);
-    }
-    return launch_gemm<Small, RESID, STK>(a, stream);
-  }
-  const int64_t tail = big_tiles % kCUs;
-  if constexpr (std::is_void_v<Wide>) {
-    return launch_gemm<Big, RESID, STK>(a, stream);
-  } else {
-    if (tail == 0 || tail > kMaxTail) return launch_gemm<Big, RESID, STK>(a, stream);
-    const int st = launch_gemm<Big, RESID, STK>(a, stream, big_tiles - tail);
-    if (st) return st;
-    return launch_tail<Wide, RESID, STK>(a, stream, big_tiles - tail);
-  }
+// 0.6% slower.)
+constexpr int64_t kCUs = 256, kMaxTail = 64;
+
+static int64_t tiles_of(const GemmArgs &a, int64_t bm, int64_t bn) {
+  return ((a.M + bm - 1) / bm) * ((a.Ncols + bn - 1) / bn);
+}
+
+// At least 256 tiles of 256x256: whole rounds of them, and a short tail as quarters of Q.
+template <class Big, class Q, bool RESID = false, int STK = 0>
+static int launch_rounds(GemmArgs &a, hipStream_t stream) {
+  const int64_t big = tiles_of(a, 256, 256), tail = big % kCUs;
+  if (tail == 0 || tail > kMaxTail) return launch_gemm<Big, RESID, STK>(a, stream);
+  const int st = launch_gemm<Big, RESID, STK>(a, stream, big - tail);
+  if (st) return st;
+  return launch_tail<Q, RESID, STK>(a, stream, big - tail);
+}
+
+// NT tile choice. Every output keeps the same k order and MFMA sequence in all tile sizes, so the
+// result is the same bit for bit. What decides is how evenly one round of tiles fills the 256 CUs;
+// measured on MI355X (us, cold launches with two rank-64 segments, ~8 us of them launch and event
+// time; before: 128x128 tiles of 8 waves up to 256 of them, else of 4 waves, below 256 tiles of
+// 256x256):
+//   M x N x K             tiles of 128x128  before  64x64  128x128  128x256  256x256
+//   512 x 1536 x 1536            48         21.0    14.7    20.2       -       34
+//   512 x 1536 x 8960            48         80.4    46.5    72         -      132
+//   1024 x 1536 x 8960           96         82      58      72         -      133
+//   1024 x 3072 x 3072          192         35.2    36      32.2       -       54
+//   2048 x 1536 x 8960          192         80.7    87      73.4       -      134
+//   3120 x 1536 x 8960          300        125       -      160       110     131
+//   4680 x 1536 x 1536          444         29.6     -       37        28.4    33.8
+//   4680 x 1536 x 8960          444        145       -      171       127     165
+//   6240 x 1536 x 1536          588         46       -       53        50      34.7
+//   9360 x 1536 x 8960          888        304       -      361       260     187
+//   4680 x 3072 x 3072          888        100       -      125        94      72
+// * up to 128 tiles of 128x128: 64x64 tiles (at most 512, two per CU);
+// * up to 256: 128x128, one per CU;
+// * while 128x256 or 256x128 tiles (whichever are fewer) fit one round: those;
+// * else 256x256, in one partly filled round or (from 256 tiles on) whole rounds and a tail.
+template <bool RESID = false, int STK = 0>
+static int dispatch_nt(GemmArgs &a, hipStream_t stream) {
+  if (tiles_of(a, 256, 256) >= kCUs) return launch_rounds<CfgNT256, CfgNT128, RESID, STK>(a, stream);
+  const int64_t mid = tiles_of(a, 128, 128);
+  if (mid <= kCUs / 2) return launch_gemm<CfgNT64, RESID, STK>(a, stream);
+  if (mid <= kCUs) return launch_gemm<CfgNT128, RESID, STK>(a, stream);
+  const int64_t wide = tiles_of(a, 128, 256), tall = tiles_of(a, 256, 128);
+  if (wide <= kCUs && wide <= tall) return launch_gemm<CfgNT128x256, RESID, STK>(a, stream);
+  if (tall <= kCUs) return launch_gemm<CfgNT256x128, RESID, STK>(a, stream);
+  return launch_gemm<CfgNT256, RESID, STK>(a, stream);
+}
+
+// NN: 8-wave 128x128 tiles while one round of them fits, 4-wave ones (two workgroups per CU) while two
+// do, else the interleaved 256x256 tile (a partly filled round below 256 of them). 6240 x 1536,
+// K = 8960: 256x256 181 us, 4-wave 128x128 252; 4680 rows: 183 and 137.
+static int dispatch_nn(GemmArgs &a, hipStream_t stream) {
+  if (tiles_of(a, 256, 256) >= kCUs) return launch_rounds<CfgNN256, CfgNN128W>(a, stream);
+  const int64_t mid = tiles_of(a, 128, 128);
+  if (mid <= kCUs) return launch_gemm<CfgNN128W>(a, stream);
+  if (mid <= 2 * kCUs) return launch_gemm<CfgNN128>(a, stream);
+  return launch_gemm<CfgNN256>(a, stream);
+}
+
+// e4m3: 64x64 tiles up to 128 of 128x128 (512 x 1536, K = 8960: 34 us, 128x128 51), 4-wave 128x128
+// tiles while two of them per CU hold the grid, else 256x256 (6240 x 1536, K = 8960: 88 us, 128x128
+// 112; from 256 tiles on with the tail as 256x256 tiles: 8-wave quarters measured 1% slower).
+static int dispatch_f8(GemmArgs &a, hipStream_t stream) {
+  const int64_t mid = tiles_of(a, 128, 128);
+  if (mid <= kCUs / 2) return launch_gemm<CfgF864>(a, stream);
+  if (mid <= 2 * kCUs) return launch_gemm<CfgF8128>(a, stream);
+  return launch_gemm<CfgF8256>(a, stream);
 }
 
 static int fill_common(GemmArgs &a, int64_t M, int64_t Kc, int64_t Ncols, const void *e, int64_t lde,
@@ -1433,7 +1545,7 @@ extern "C" int mlora_gemm_fwd(const void *x, int64_t ldx, int64_t M, int64_t K, 
   a.Y = static_cast<uint16_t *>(y);
   a.ldy = ldy;
   a.accumulate = accumulate ? 1 : 0;
-  return dispatch_gemm<CfgNT256, CfgNT128>(a, static_cast<hipStream_t>(stream));
+  return dispatch_nt(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlora_gemm_fwd_stacked(const void *x, int64_t ldx, int64_t M, int64_t K, const void *w, int64_t ldw,
@@ -1476,7 +1588,7 @@ extern "C" int mlora_gemm_fwd_stacked(const void *x, int64_t ldx, int64_t M, int
   a.group_cols = (int32_t)group_cols;
   a.group_ecols = (int32_t)group_ecols;
   for (int64_t g = 0; g < groups; ++g) a.Yg[g] = static_cast<uint16_t *>(y_ptrs[g]);
-  return dispatch_gemm<CfgNT256, CfgNT128, false, 1>(a, static_cast<hipStream_t>(stream));
+  return dispatch_nt<false, 1>(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlora_gemm_dx_stacked(const void *const *dy_ptrs, int64_t lddy, int64_t M, int64_t group_cols,
@@ -1511,7 +1623,7 @@ extern "C" int mlora_gemm_dx_stacked(const void *const *dy_ptrs, int64_t lddy, i
   a.groups = (int32_t)groups;
   a.group_cols = (int32_t)group_cols;
   for (int64_t g = 0; g < groups; ++g) a.Pg[g] = static_cast<const uint16_t *>(dy_ptrs[g]);
-  return dispatch_gemm<CfgNT256, CfgNT128, false, 2>(a, static_cast<hipStream_t>(stream));
+  return dispatch_nt<false, 2>(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlora_gemm_fwd_gated(const void *x, int64_t ldx, int64_t M, int64_t K, const void *w, int64_t ldw,
@@ -1565,7 +1677,7 @@ extern "C" int mlora_gemm_fwd_gated(const void *x, int64_t ldx, int64_t M, int64
   a.ldgate = ldgate;
   a.gate_rows = (int32_t)gate_rows;
   a.res_f32 = f32 ? 1 : 0;
-  return dispatch_gemm<CfgNT256, CfgNT128, true>(a, static_cast<hipStream_t>(stream));
+  return dispatch_nt<true>(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlora_gemm_dx(const void *dy, int64_t lddy, int64_t M, int64_t N, const void *w, int64_t ldw, int64_t K,
@@ -1592,7 +1704,7 @@ extern "C" int mlora_gemm_dx(const void *dy, int64_t lddy, int64_t M, int64_t N,
   a.Y = static_cast<uint16_t *>(dx);
   a.ldy = lddx;
   a.accumulate = accumulate ? 1 : 0;
-  return dispatch_gemm<CfgNN256, CfgNN128>(a, static_cast<hipStream_t>(stream));
+  return dispatch_nn(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlora_gemm_fwd_fp8(const void *xq, int64_t ldx, const float *x_scale, int64_t M, int64_t K,
@@ -1627,5 +1739,5 @@ extern "C" int mlora_gemm_fwd_fp8(const void *xq, int64_t ldx, const float *x_sc
   a.Y = static_cast<uint16_t *>(y);
   a.ldy = ldy;
   a.accumulate = accumulate ? 1 : 0;
-  return dispatch_gemm<CfgF8256, CfgF8128>(a, static_cast<hipStream_t>(stream));
+  return dispatch_f8(a, static_cast<hipStream_t>(stream));
 }
