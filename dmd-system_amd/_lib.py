@@ -75,6 +75,8 @@ SIGNATURES = {
     "mlora_div_rows_bf16_batch": (_int, [_pvp, _pi64, _vp, _i64, _pi64, _pvp, _pi64, _i32, _vp]),
     "mlora_gemm_fwd_fp8": (_int, [_vp, _i64, _vp, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _int, _vp, _i64,
                                   _pvp, _pi32, _i32, _pi64, _pi32, _i32, _vp, _i64, _int, _vp]),
+    "mlora_prepare_operands": (_int, [_pvp, _int, _pi64, _pi64, _pi64, _pi64, _pi64, _pvp, _pvp, _pi64, _pvp, _pi64,
+                                      _i32, _vp]),
     "mlora_f32_shrink": (_int, [_vp, _i64, _i64, _i64, _pvp, _int, _pi32, _pf32, _i32,
                                 _pi64, _pi32, _i32, _vp, _i64, _i64, _vp]),
     "mlora_f32_gemm_fwd": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,

@@ -620,6 +620,60 @@ def gemm_fwd_fp8(xq: torch.Tensor, x_scale: torch.Tensor, wq: torch.Tensor, w_sc
 
 # ------------------------------------------------------------ fp32 arithmetic
 
+def prepare_operands(srcs: Sequence[torch.Tensor], *, hi: Sequence[torch.Tensor | None] | None = None,
+                     lo: Sequence[torch.Tensor | None] | None = None,
+                     t: Sequence[torch.Tensor | None] | None = None) -> None:
+    """Fills hi[i] = bf16(srcs[i]), lo[i] = bf16(srcs[i] - hi[i]) and t[i] = hi[i] transposed, all matrices in
+    one launch; the outputs are bf16 row-major views (of one padded shape per matrix: rows and columns
+    past srcs[i]'s are zeros). The sources share one dtype, bf16 or float32."""
+    if not srcs:
+        return
+    n = len(srcs)
+    dt = srcs[0].dtype
+    hi, lo, t = hi or [None] * n, lo or [None] * n, t or [None] * n
+    pr, pc, old, tld = [], [], [], []
+    for i, s in enumerate(srcs):
+        _require(s.is_cuda and s.dtype == dt and dt in _DT and s.dim() == 2 and (s.stride(1) == 1 or s.shape[1] <= 1),
+                 "operand sources are row-major bf16 or float32 device matrices of one dtype")
+        shape = ld = None
+        for name, o in (("hi", hi[i]), ("lo", lo[i])):
+            if o is not None:
+                _check_rows("operand " + name, o)
+                _require(shape is None or (shape == o.shape and ld == o.stride(0)), "hi and lo share shape and pitch")
+                shape, ld = o.shape, o.stride(0)
+        if t[i] is not None:
+            _check_rows("operand t", t[i])
+            _require(shape is None or tuple(shape) == (t[i].shape[1], t[i].shape[0]), "t has hi's shape transposed")
+            shape = shape or (t[i].shape[1], t[i].shape[0])
+        _require(shape is not None and shape[0] >= s.shape[0] and shape[1] >= s.shape[1], "an output of padded shape")
+        pr.append(shape[0])
+        pc.append(shape[1])
+        old.append(ld or 0)
+        tld.append(t[i].stride(0) if t[i] is not None else 0)
+    lib, i64, ptrs = _lib.load(), _lib.i64_array, _lib.ptr_array
+    _lib.check("mlora_prepare_operands", lib.mlora_prepare_operands(
+        ptrs([s.data_ptr() for s in srcs]), _DT[dt], i64([s.stride(0) for s in srcs]), i64([s.shape[0] for s in srcs]),
+        i64([s.shape[1] for s in srcs]), i64(pr), i64(pc), ptrs([_ptr(o) for o in hi]), ptrs([_ptr(o) for o in lo]),
+        i64(old), ptrs([_ptr(o) for o in t]), i64(tld), n, _stream(srcs[0])))
+
+
+def transpose_many(mats: Sequence[torch.Tensor]) -> list[torch.Tensor]:
+    """The contiguous bf16 matrices transposed ([c, r] contiguous each), in one launch."""
+    outs = [torch.empty((m.shape[1], m.shape[0]), dtype=torch.bfloat16, device=m.device) for m in mats]
+    if not mats:
+        return outs
+    for m in mats:
+        _check_rows("operand", m)
+        _require(m.is_contiguous(), "operands to transpose are contiguous")
+    n, lib = len(mats), _lib.load()
+    none, zero = _lib.ptr_array([None] * n), _lib.i64_array([0] * n)
+    rows, cols = _lib.i64_array([m.shape[0] for m in mats]), _lib.i64_array([m.shape[1] for m in mats])
+    _lib.check("mlora_prepare_operands", lib.mlora_prepare_operands(
+        _lib.ptr_array([m.data_ptr() for m in mats]), _lib.BF16, cols, rows, cols, rows, cols, none, none, zero,
+        _lib.ptr_array([o.data_ptr() for o in outs]), rows, n, _stream(mats[0])))
+    return outs
+
+
 def split_hi_lo(t: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """(hi, lo) bf16 parts of a float matrix: hi = bf16(t), lo = bf16(t - hi), both contiguous.
     hi + lo carries ~16 significant bits of t (relative error <= 2^-16)."""

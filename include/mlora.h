@@ -415,6 +415,18 @@ int mlora_gemm_fwd_fp8(const void *xq, int64_t ldx, const float *x_scale, int64_
                        void *y, int64_t ldy, int accumulate,
                        void *stream);
 
+/* Adapter operands of one call, every matrix in one launch (64 per launch): matrix i, src[i]
+ * [rows, cols] (bf16 or float32, pitch src_ld), zero-padded to [padded_rows, padded_cols], as
+ *   hi[i] = bf16(v) and lo[i] = bf16(v - hi) [padded_rows, padded_cols] (pitch out_ld), and
+ *   t[i]  = hi transposed [padded_cols, padded_rows] (pitch t_ld);
+ * any of the three may be NULL. Host arrays of n entries. */
+int mlora_prepare_operands(const void *const *src, int src_dtype, const int64_t *src_ld,
+                           const int64_t *rows, const int64_t *cols,
+                           const int64_t *padded_rows, const int64_t *padded_cols,
+                           void *const *hi, void *const *lo, const int64_t *out_ld,
+                           void *const *t, const int64_t *t_ld, int32_t n,
+                           void *stream);
+
 /* ---- fp32 arithmetic (the reference's precision='fp32' mode: no autocast,
  * training/single_device.py:77-80, so TrainableLowRankLinear computes
  * base(x) + s·F.linear(F.linear(x, A), B) and its autograd backward in fp32,

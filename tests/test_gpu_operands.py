@@ -1,0 +1,42 @@
+"""Adapter operands made in one launch (hi / lo parts, padding, stacking, transposes) against the
+torch conversions, bit for bit: both are defined roundings. Shapes at the edges of the 64x64 tiles, more
+matrices than one launch takes, outputs inside wider buffers, special values."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(t):
+    return t.contiguous().view(torch.int16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pad", [8, 3])  # 16-byte accesses, and rows that do not allow them
+@pytest.mark.parametrize("shapes", [[(8, 8)], [(128, 1536), (72, 72)], [(64, 64), (65, 63), (1, 129), (0, 16)], [(5, 200)] * 70])
+def test_prepared_operands_are_the_torch_conversions(pkg, dev, dtype, shapes, pad):
+    k = pkg.kernels
+    g = torch.Generator().manual_seed(len(shapes))
+    srcs, his, los, ts = [], [], [], []
+    for i, (r, c) in enumerate(shapes):
+        wide = (torch.randn(r, c + pad, generator=g) * 10.0 ** (i % 7 - 3)).to(dev, dtype)
+        if r:
+            wide[0, 0] = [float("inf"), float("-inf"), 0.0, 1e-40, -0.0][i % 5]
+        srcs.append(wide[:, :c])
+        pr, pc = (r + 7) // 8 * 8, (c + 7) // 8 * 8
+        hi, lo, t = (torch.full(s, -1.0, dtype=torch.bfloat16, device=dev) for s in ((pr, pc + 8), (pr, pc + 8), (pc, pr + pad)))
+        his.append(hi[:, :pc])
+        los.append(lo[:, :pc])
+        ts.append(t[:, :pr])
+    k.prepare_operands(srcs, hi=his, lo=los, t=ts)
+    for s, hi, lo, t in zip(srcs, his, los, ts):
+        r, c = s.shape
+        want = torch.zeros(hi.shape, dtype=torch.bfloat16, device=dev)
+        want_lo = torch.zeros_like(want)
+        want[:r, :c] = s.to(torch.bfloat16)
+        want_lo[:r, :c] = (s.float() - want[:r, :c].float()).to(torch.bfloat16)
+        finite = torch.isfinite(want.float())  # inf - inf: not a number on both sides, of any payload
+        assert torch.equal(bits(hi), bits(want)) and torch.equal(bits(t), bits(want.t()))
+        assert torch.equal(lo[finite], want_lo[finite])
+    outs = k.transpose_many([h.contiguous() for h in his])
+    assert all(torch.equal(bits(o), bits(h.t())) for o, h in zip(outs, his))
