@@ -140,20 +140,31 @@ def check(name: str, status: int) -> None:
         raise MloraError(name, status, msg)
 
 
+_ARRAYS: dict = {}  # (element type, length) -> array type
+
+
+def _array(ctype, values) -> ctypes.Array:
+    n = len(values) or 1
+    t = _ARRAYS.get((ctype, n))
+    if t is None:
+        t = _ARRAYS[(ctype, n)] = ctype * n
+    return t(*values)
+
+
 def ptr_array(values) -> ctypes.Array:
-    return (ctypes.c_void_p * max(1, len(values)))(*[v or None for v in values])
+    return _array(ctypes.c_void_p, values)
 
 
 def i32_array(values) -> ctypes.Array:
-    return (ctypes.c_int32 * max(1, len(values)))(*values)
+    return _array(ctypes.c_int32, values)
 
 
 def i64_array(values) -> ctypes.Array:
-    return (ctypes.c_int64 * max(1, len(values)))(*values)
+    return _array(ctypes.c_int64, values)
 
 
 def f32_array(values) -> ctypes.Array:
-    return (ctypes.c_float * max(1, len(values)))(*values)
+    return _array(ctypes.c_float, values)
 
 
 def python_source_hash() -> str:

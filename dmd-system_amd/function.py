@@ -27,6 +27,7 @@ The adapter gradients come back in the parameters' dtype (fp32 masters stay fp32
 """
 from __future__ import annotations
 
+import contextlib
 from typing import Sequence
 
 import torch
@@ -140,7 +141,7 @@ def _prepare(ctx, x, N: int, ab, scales, routing: SegmentRouting, grad0: int, ro
     A_ops, B_ops = [a for a, _ in A], [b for b, _ in B]
     A_lo, B_lo = ([a for _, a in A], [b for _, b in B]) if split else ([], [])
     width = kernels.padded_rank(pranks)
-    need_b_grad = any(ctx.needs_input_grad[grad0 + n + i] for i in range(n))
+    need_b_grad = any(ctx.needs_input_grad[grad0 + n:grad0 + 2 * n])
     h_rows, h_frag = (None, [])
     if width > 0:
         h_rows, h_frag = kernels.shrink(x, A_ops, 0, scales, routing, want_frag=need_b_grad, width=width,
@@ -171,10 +172,8 @@ def _backward(ctx, dy, x, dx_gemm, A_ops, B_ops, h_frag, B_lo=None, row_div=None
     dy is bf16 contiguous; g_rows (the LoRA term of dX) are divided by row_div
     when given (the e4m3 dX folds dY's row scale into them). B_lo: the lo parts of
     split fp32 masters (g then uses hi + lo)."""
-    n, g0, routing = ctx.n, ctx.grad0, ctx.routing
-    need_x = ctx.needs_input_grad[0]
-    need_a = [ctx.needs_input_grad[g0 + i] for i in range(n)]
-    need_b = [ctx.needs_input_grad[g0 + n + i] for i in range(n)]
+    n, g0, routing, need = ctx.n, ctx.grad0, ctx.routing, ctx.needs_input_grad
+    need_x, need_a, need_b = need[0], need[g0:g0 + n], need[g0 + n:g0 + 2 * n]
     dx = None
     g_rows = g_frag = None
     if ctx.width > 0 and (need_x or any(need_a)):
@@ -187,13 +186,13 @@ def _backward(ctx, dy, x, dx_gemm, A_ops, B_ops, h_frag, B_lo=None, row_div=None
     if any(need_b):
         outs = kernels.seg_outer(dy, h_frag, ctx.width, ctx.pranks, routing, 0,
                                  [ctx.b_dtypes[i] for i in range(n)])
-        dBs = [o[:, :r] if nb else None for o, r, nb in zip(outs, ctx.ranks, need_b)]
+        dBs = [(o if o.shape[1] == r else o[:, :r]) if nb else None for o, r, nb in zip(outs, ctx.ranks, need_b)]
     if need_x:
         dx = dx_gemm(g_rows)
     if any(need_a):
         outs = kernels.seg_outer(x, g_frag, ctx.width, ctx.pranks, routing, 1,
                                  [ctx.a_dtypes[i] for i in range(n)])
-        dAs = [o[:r] if na else None for o, r, na in zip(outs, ctx.ranks, need_a)]
+        dAs = [(o if o.shape[0] == r else o[:r]) if na else None for o, r, na in zip(outs, ctx.ranks, need_a)]
     return dx, dAs, dBs
 
 
@@ -636,7 +635,7 @@ class StackedLinearsFunction(torch.autograd.Function):
 
 def _bf16_rows(x: torch.Tensor, weight_dtype: torch.dtype) -> torch.Tensor:
     """x [..., K] as contiguous bf16 rows [M, K] (under bf16 autocast the cast is done here)."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
         weight_dtype = torch.bfloat16
@@ -671,19 +670,34 @@ def shared_input_multi_lora(x: torch.Tensor, weights: Sequence[torch.Tensor], bi
         N = next(iter(widths))
         want_t = transposed_base_for_dx and torch.is_grad_enabled() and x.requires_grad
         w_cat, b_cat, w_cat_t = stacked_bases(list(weights), list(biases), want_t)
-        with torch.autocast("cuda", enabled=False):
+        with _no_autocast():
             ys = StackedLinearsFunction.apply(x2, routing, tuple(scales), G, w_cat, b_cat, w_cat_t if want_t else None,
                                               split, *flat_a, *flat_b)
-        return tuple(v.reshape(*lead, N) for v in ys)
+        return tuple(_unrows(v, lead) for v in ys)
     ws = tuple(w.detach().to(torch.bfloat16) for w in weights)  # a no-op unless autocast runs fp32 bases
     bs = tuple(None if b is None else b.detach() for b in biases)
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         ys = SharedInputMultiLoRAFunction.apply(x2, routing, tuple(scales), G, ws, bs, split, *flat_a, *flat_b)
-    return tuple(y.reshape(*lead, w.shape[0]) for y, w in zip(ys, ws))
+    return tuple(_unrows(y, lead) for y in ys)
 
 
 def _autocast_bf16() -> bool:
     return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """t [..., K] as rows [M, K] (a matrix stays itself: no view node in the graph)."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
+def _unrows(y: torch.Tensor, lead) -> torch.Tensor:
+    """Rows [M, N] as [*lead, N]."""
+    return y if len(lead) == 1 else y.reshape(*lead, y.shape[-1])
+
+
+def _no_autocast():
+    """The op runs outside autocast (a context only where one is active: it costs more than a launch)."""
+    return torch.autocast("cuda", enabled=False) if torch.is_autocast_enabled("cuda") else contextlib.nullcontext()
 
 
 def multi_lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
@@ -699,7 +713,7 @@ def multi_lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor 
     out computed in float32 (MultiLoRAF32Function). Other combinations raise."""
     K = x.shape[-1]
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
+    x2 = _rows(x)
     split = f32 = False
     if _autocast_bf16():
         x2 = x2.to(torch.bfloat16)
@@ -717,14 +731,14 @@ def multi_lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor 
                            "base weight, or call it under torch.autocast('cuda', dtype=torch.bfloat16)")
     if not x2.is_cuda:
         raise RuntimeError("multi-LoRA linear runs on the ROCm device only (HIP kernels, no CPU path)")
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         if f32:
             y = MultiLoRAF32Function.apply(x2.contiguous(), weight.detach().contiguous(), bias, routing,
                                            tuple(scales), *lora_as, *lora_bs)
         else:
             y = MultiLoRAFunction.apply(x2.contiguous(), weight, weight_t, bias, routing, tuple(scales), split,
                                         *lora_as, *lora_bs)
-    return y.reshape(*lead, weight.shape[0])
+    return _unrows(y, lead)
 
 
 def multi_lora_linear_gated(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
@@ -746,10 +760,10 @@ def multi_lora_linear_gated(x: torch.Tensor, weight: torch.Tensor, bias: torch.T
     g2 = gate.reshape(-1, N)
     if g2.stride(1) != 1 or g2.stride(0) % 4 or g2.data_ptr() % 16:
         g2 = g2.contiguous()
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         out = MultiLoRAGatedResidualFunction.apply(x2, weight, weight_t, bias, routing, tuple(scales),
-                                                   residual.reshape(-1, N).contiguous(), g2, *lora_as, *lora_bs)
-    return out.reshape(*lead, N)
+                                                   _rows(residual).contiguous(), g2, *lora_as, *lora_bs)
+    return _unrows(out, lead)
 
 
 def multi_lora_linear_fp8(x: torch.Tensor, wq: torch.Tensor, w_scale: torch.Tensor, bias: torch.Tensor | None,
@@ -763,7 +777,7 @@ def multi_lora_linear_fp8(x: torch.Tensor, wq: torch.Tensor, w_scale: torch.Tens
     the dequantised base (no quantisation of dY; +16-17% per fwd+bwd step at config 5)."""
     K = x.shape[-1]
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, K)
+    x2 = _rows(x)
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
     if x2.dtype != torch.bfloat16:
@@ -773,7 +787,7 @@ def multi_lora_linear_fp8(x: torch.Tensor, wq: torch.Tensor, w_scale: torch.Tens
         raise RuntimeError("multi-LoRA linear runs on the ROCm device only (HIP kernels, no CPU path)")
     if wq_t is None and not dx_bf16:
         wq_t = wq.t().contiguous()
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         y = MultiLoRAFP8Function.apply(x2.contiguous(), wq, w_scale, wq_t, bias, routing, tuple(scales),
                                        bool(dx_bf16), *lora_as, *lora_bs)
-    return y.reshape(*lead, wq.shape[0])
+    return _unrows(y, lead)

@@ -6,7 +6,7 @@ missing library raise.
 """
 from __future__ import annotations
 
-import ctypes
+import functools
 from typing import Sequence
 
 import torch
@@ -22,24 +22,28 @@ def _require(cond: bool, message: str) -> None:
         raise RuntimeError("multi-LoRA kernel contract: " + message)
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def _stream(t: torch.Tensor) -> int:
+    """The current stream's handle on t's device (without building a torch.cuda.Stream)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _row_ptr(t: torch.Tensor, row: int) -> int:
+    """Address of row `row` of a row-major matrix."""
+    return t.data_ptr() + (row * t.stride(0) * t.element_size() if row else 0)
+
+
 def _check_rows(name: str, t: torch.Tensor, cols: int | None = None) -> None:
+    if t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1 and (cols is None or t.shape[1] == cols):
+        return
     _require(t.is_cuda, f"{name} must be a ROCm device tensor")
     _require(t.dtype == torch.bfloat16, f"{name} must be bfloat16, got {t.dtype}")
     _require(t.dim() == 2 and t.stride(1) == 1, f"{name} must be a 2-D row-major matrix")
     if cols is not None:
         _require(t.shape[1] == cols, f"{name} has {t.shape[1]} columns, expected {cols}")
-
-
-def _routing_arrays(off, ids):
-    return _lib.i64_array(off), _lib.i32_array(ids), len(ids)
 
 
 def padded_rank(ranks: Sequence[int]) -> int:
@@ -55,16 +59,27 @@ def frag_jtiles(width: int) -> int:
 _FRAG_TILE_BYTES = 2 * 64 * 16  # one j-tile (hi + lo) of one 32-row block in the fragment layout
 
 
+# Sizes that depend on the call's integers alone (host arithmetic of the library), by value.
+@functools.lru_cache(maxsize=512)
+def _frag_bytes(routing: SegmentRouting, group: int, jtiles: int) -> int:
+    r0, r1, o, i, n = routing.call_arrays(_lib.MAX_SEGMENTS)[group]
+    nbytes = _lib.load().mlora_frag_bytes(r1 - r0, jtiles, o, i, n)
+    _lib.check("mlora_frag_bytes", min(nbytes, 0))
+    return nbytes
+
+
+@functools.lru_cache(maxsize=512)
+def _outer_workspace(name: str, routing: SegmentRouting, group: int, C: int, ranks: tuple) -> int:
+    r0, r1, o, i, n = routing.call_arrays(_lib.MAX_SEGMENTS)[group]
+    nbytes = getattr(_lib.load(), name)(r1 - r0, C, _lib.i32_array(ranks), len(ranks), o, i, n)
+    _lib.check(name, min(nbytes, 0))
+    return nbytes
+
+
 def alloc_frags(routing: SegmentRouting, jtiles: int, device) -> list:
     """Empty hi/lo fragment buffers (one per call group of `routing`) of `jtiles` j-tiles."""
-    lib = _lib.load()
-    out = []
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
-        o, i, n = _routing_arrays(off, ids)
-        nbytes = lib.mlora_frag_bytes(r1 - r0, jtiles, o, i, n)
-        _lib.check("mlora_frag_bytes", nbytes if nbytes < 0 else 0)
-        out.append(torch.empty(max(nbytes, 16) // 2, dtype=torch.bfloat16, device=device))
-    return out
+    return [torch.empty(max(_frag_bytes(routing, g, jtiles), 16) // 2, dtype=torch.bfloat16, device=device)
+            for g in range(len(routing.call_arrays(_lib.MAX_SEGMENTS)))]
 
 
 def shrink(p: torch.Tensor, ops: Sequence[torch.Tensor], op_layout: int, scales: Sequence[float],
@@ -104,7 +119,7 @@ def shrink(p: torch.Tensor, ops: Sequence[torch.Tensor], op_layout: int, scales:
         _require(h_out.shape[0] == M and h_out.shape[1] >= max([0, *ranks]), "h_out is [M, >= max rank]")
     h_rows = h_out if h_out is not None else torch.empty((M, width), dtype=torch.bfloat16, device=p.device)
     lib = _lib.load()
-    ptrs, rk, sc = _lib.ptr_array([_ptr(o) for o in ops]), _lib.i32_array(ranks), _lib.f32_array(scales)
+    ptrs, rk, sc = _lib.ptr_array([t.data_ptr() for t in ops]), _lib.i32_array(ranks), _lib.f32_array(scales)
     lo_ptrs = None if ops_lo is None else _lib.ptr_array([_ptr(o) for o in ops_lo])
     jt = frag_jtiles(width) if frag_jt is None else frag_jt
     _require(0 <= frag_t0 and frag_t0 * 16 + max([0, *ranks]) <= jt * 16, "fragment j-tiles out of range")
@@ -112,16 +127,15 @@ def shrink(p: torch.Tensor, ops: Sequence[torch.Tensor], op_layout: int, scales:
     frags = None
     if want_frag:
         frags = frag_out if frag_out is not None else alloc_frags(routing, jt, p.device)
-        _require(len(frags) == len(list(routing.groups(_lib.MAX_SEGMENTS))), "one fragment buffer per call group")
-    for g, (r0, r1, off, ids) in enumerate(routing.groups(_lib.MAX_SEGMENTS)):
-        o, i, n = _routing_arrays(off, ids)
+        _require(len(frags) == len(routing.call_arrays(_lib.MAX_SEGMENTS)), "one fragment buffer per call group")
+    for g, (r0, r1, o, i, n) in enumerate(routing.call_arrays(_lib.MAX_SEGMENTS)):
         fptr = None if frags is None else frags[g].data_ptr() + frag_t0 * _FRAG_TILE_BYTES
         if r1 == r0:
             continue
         _lib.check("mlora_shrink", lib.mlora_shrink(
-            p[r0:r1].data_ptr(), p.stride(0), r1 - r0, K, ptrs, lo_ptrs, op_layout, rk, sc, len(ops),
-            o, i, n, h_rows[r0:r1].data_ptr(), h_rows.stride(0), fptr, jt,
-            None if row_div is None else row_div[r0:r1].data_ptr(), stream))
+            _row_ptr(p, r0), p.stride(0), r1 - r0, K, ptrs, lo_ptrs, op_layout, rk, sc, len(ops),
+            o, i, n, _row_ptr(h_rows, r0), h_rows.stride(0), fptr, jt,
+            None if row_div is None else _row_ptr(row_div, r0), stream))
     return h_rows, frags
 
 
@@ -143,18 +157,17 @@ def gemm_fwd(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, h_rows
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _check_rows("Y", y, N)
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(b) for b in bs]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([b.data_ptr() for b in bs]), _lib.i32_array(ranks)
     ldh = h_rows.stride(0) if h_rows is not None else 0
     stream = _stream(x)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
-        hr = None if h_rows is None else h_rows[r0:r1].data_ptr()
+        hr = None if h_rows is None else _row_ptr(h_rows, r0)
         _lib.check("mlora_gemm_fwd", lib.mlora_gemm_fwd(
-            x[r0:r1].data_ptr(), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N,
+            _row_ptr(x, r0), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N,
             _ptr(bias), _DT[bias.dtype] if bias is not None else 0, hr, ldh,
-            ptrs, rk, len(bs), o, i, n, y[r0:r1].data_ptr(), y.stride(0), int(accumulate), stream))
+            ptrs, rk, len(bs), o, i, n, _row_ptr(y, r0), y.stride(0), int(accumulate), stream))
     return y
 
 
@@ -181,15 +194,14 @@ def gemm_fwd_stacked(x: torch.Tensor, w_cat: torch.Tensor, bias_cat: torch.Tenso
     ptrs, rk = _lib.ptr_array([_ptr(b) for b in bs_cat]), _lib.i32_array(ranks)
     ldh = h_rows.stride(0) if h_rows is not None else 0
     stream = _stream(x)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
-        hr = None if h_rows is None else h_rows[r0:r1].data_ptr()
+        hr = None if h_rows is None else _row_ptr(h_rows, r0)
         _lib.check("mlora_gemm_fwd_stacked", lib.mlora_gemm_fwd_stacked(
-            x[r0:r1].data_ptr(), x.stride(0), r1 - r0, K, w_cat.data_ptr(), w_cat.stride(0), NT, group_cols,
+            _row_ptr(x, r0), x.stride(0), r1 - r0, K, w_cat.data_ptr(), w_cat.stride(0), NT, group_cols,
             _ptr(bias_cat), _DT[bias_cat.dtype] if bias_cat is not None else 0, hr, ldh, group_ecols,
-            ptrs, rk, len(bs_cat), o, i, n, _lib.ptr_array([y[r0:r1].data_ptr() for y in ys]), group_cols, stream))
+            ptrs, rk, len(bs_cat), o, i, n, _lib.ptr_array([_row_ptr(y, r0) for y in ys]), group_cols, stream))
     return ys
 
 
@@ -214,14 +226,13 @@ def gemm_dx_stacked(dys: Sequence[torch.Tensor], w_cat_t: torch.Tensor, g_rows: 
     ptrs, rk = _lib.ptr_array([_ptr(a) for a in a_t_cat]), _lib.i32_array(ranks)
     ldg = g_rows.stride(0) if g_rows is not None else 0
     stream = _stream(dys[0])
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
         _lib.check("mlora_gemm_dx_stacked", lib.mlora_gemm_dx_stacked(
-            _lib.ptr_array([d[r0:r1].data_ptr() for d in dys]), dys[0].stride(0), r1 - r0, N, G,
-            w_cat_t.data_ptr(), w_cat_t.stride(0), K, None if g_rows is None else g_rows[r0:r1].data_ptr(), ldg,
-            ptrs, rk, len(a_t_cat), o, i, n, dx[r0:r1].data_ptr(), dx.stride(0), stream))
+            _lib.ptr_array([_row_ptr(d, r0) for d in dys]), dys[0].stride(0), r1 - r0, N, G,
+            w_cat_t.data_ptr(), w_cat_t.stride(0), K, None if g_rows is None else _row_ptr(g_rows, r0), ldg,
+            ptrs, rk, len(a_t_cat), o, i, n, _row_ptr(dx, r0), dx.stride(0), stream))
     return dx
 
 
@@ -265,20 +276,19 @@ def gemm_fwd_gated(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
     _check_stream("out", y, N)
     _require(y.dtype == res.dtype, "out has the residual stream's dtype")
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(b) for b in bs]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([b.data_ptr() for b in bs]), _lib.i32_array(ranks)
     ldh = h_rows.stride(0) if h_rows is not None else 0
     stream = _stream(x)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
         _require(r0 % per == 0, "a call group must start at a gate-row boundary")
-        o, i, n = _routing_arrays(off, ids)
-        hr = None if h_rows is None else h_rows[r0:r1].data_ptr()
+        hr = None if h_rows is None else _row_ptr(h_rows, r0)
         _lib.check("mlora_gemm_fwd_gated", lib.mlora_gemm_fwd_gated(
-            x[r0:r1].data_ptr(), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N,
+            _row_ptr(x, r0), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N,
             _ptr(bias), _DT[bias.dtype] if bias is not None else 0, hr, ldh,
-            ptrs, rk, len(bs), o, i, n, res[r0:r1].data_ptr(), res.stride(0),
-            gate[r0 // per:].data_ptr(), gate.stride(0), per, y[r0:r1].data_ptr(), y.stride(0), _DT[res.dtype],
+            ptrs, rk, len(bs), o, i, n, _row_ptr(res, r0), res.stride(0),
+            gate[r0 // per:].data_ptr(), gate.stride(0), per, _row_ptr(y, r0), y.stride(0), _DT[res.dtype],
             stream))
     return y
 
@@ -442,17 +452,16 @@ def gemm_dx(dy: torch.Tensor, w: torch.Tensor, g_rows: torch.Tensor | None, as_:
     dx = out if out is not None else torch.empty((M, K), dtype=torch.bfloat16, device=dy.device)
     _check_rows("dX", dx, K)
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(a) for a in as_]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([a.data_ptr() for a in as_]), _lib.i32_array(ranks)
     ldg = g_rows.stride(0) if g_rows is not None else 0
     stream = _stream(dy)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
-        gr = None if g_rows is None else g_rows[r0:r1].data_ptr()
+        gr = None if g_rows is None else _row_ptr(g_rows, r0)
         _lib.check("mlora_gemm_dx", lib.mlora_gemm_dx(
-            dy[r0:r1].data_ptr(), dy.stride(0), r1 - r0, N, w.data_ptr(), w.stride(0), K, gr, ldg,
-            ptrs, rk, len(as_), o, i, n, dx[r0:r1].data_ptr(), dx.stride(0), int(accumulate), stream))
+            _row_ptr(dy, r0), dy.stride(0), r1 - r0, N, w.data_ptr(), w.stride(0), K, gr, ldg,
+            ptrs, rk, len(as_), o, i, n, _row_ptr(dx, r0), dx.stride(0), int(accumulate), stream))
     return dx
 
 
@@ -467,7 +476,7 @@ def seg_outer(p: torch.Tensor, frags: list, width: int, ranks: Sequence[int], ro
     M, C = p.shape
     _check_rows("P", p, C)
     lib = _lib.load()
-    groups = list(routing.groups(_lib.MAX_SEGMENTS))
+    groups = routing.call_arrays(_lib.MAX_SEGMENTS)
     _require(frags is not None and len(frags) == len(groups), "h fragments from shrink() of the same routing")
     dtypes = list(out_dtypes)
     _require(all(d in _DT for d in dtypes), "adapter gradients are float32 or bfloat16")
@@ -475,23 +484,23 @@ def seg_outer(p: torch.Tensor, frags: list, width: int, ranks: Sequence[int], ro
     _require(0 <= frag_t0 and frag_t0 * 16 + max([0, *ranks]) <= jt * 16, "fragment j-tiles out of range")
     outs: list[torch.Tensor | None] = [None] * len(ranks)
     stream = _stream(p)
-    shape = (lambda r: (C, r)) if out_layout == 0 else (lambda r: (r, C))
     single = len(groups) == 1
     # Adapters are reduced per output dtype (normally one dtype for all).
     for dt in sorted(set(dtypes), key=str):
         sel = [a for a in range(len(ranks)) if dtypes[a] == dt]
-        mask_ranks = _lib.i32_array([r if dtypes[a] == dt else 0 for a, r in enumerate(ranks)])
+        masked = tuple(r if dtypes[a] == dt else 0 for a, r in enumerate(ranks))
+        mask_ranks = _lib.i32_array(masked)
+        pdt = dt if single else torch.float32
         # several row groups: reduce each into fp32, then add in group order
-        for (r0, r1, off, ids), frag in zip(groups, frags):
-            o, i, n = _routing_arrays(off, ids)
-            ws_bytes = lib.mlora_seg_outer_workspace_bytes(r1 - r0, C, mask_ranks, len(ranks), o, i, n)
-            _lib.check("mlora_seg_outer_workspace_bytes", ws_bytes if ws_bytes < 0 else 0)
+        for g, ((r0, r1, o, i, n), frag) in enumerate(zip(groups, frags)):
+            ws_bytes = _outer_workspace("mlora_seg_outer_workspace_bytes", routing, g, C, masked)
             ws = torch.empty((max(ws_bytes, 16) + 15) // 16 * 4, dtype=torch.float32, device=p.device)
-            part = [torch.empty(shape(ranks[a]), dtype=dt if single else torch.float32, device=p.device)
-                    if a in sel else None for a in range(len(ranks))]
+            part: list[torch.Tensor | None] = [None] * len(ranks)
+            for a in sel:
+                part[a] = torch.empty((C, ranks[a]) if out_layout == 0 else (ranks[a], C), dtype=pdt, device=p.device)
             _lib.check("mlora_seg_outer", lib.mlora_seg_outer(
-                p[r0:r1].data_ptr(), p.stride(0), r1 - r0, C, frag.data_ptr() + frag_t0 * _FRAG_TILE_BYTES, jt,
-                _lib.ptr_array([_ptr(t) for t in part]), out_layout, _DT[dt if single else torch.float32],
+                _row_ptr(p, r0), p.stride(0), r1 - r0, C, frag.data_ptr() + frag_t0 * _FRAG_TILE_BYTES, jt,
+                _lib.ptr_array([_ptr(t) for t in part]), out_layout, _DT[pdt],
                 mask_ranks, len(ranks), o, i, n, ws.data_ptr(), ws.numel() * 4, stream))
             for a in sel:
                 outs[a] = part[a] if outs[a] is None else outs[a] + part[a]
@@ -602,19 +611,18 @@ def gemm_fwd_fp8(xq: torch.Tensor, x_scale: torch.Tensor, wq: torch.Tensor, w_sc
         _require(b.is_contiguous() and b.shape[0] == N, "lora_b must be contiguous [N, r]")
     y = torch.empty((M, N), dtype=torch.bfloat16, device=xq.device)
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(b) for b in bs]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([b.data_ptr() for b in bs]), _lib.i32_array(ranks)
     ldh = h_rows.stride(0) if h_rows is not None else 0
     stream = _stream(xq)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
-        hr = None if h_rows is None else h_rows[r0:r1].data_ptr()
+        hr = None if h_rows is None else _row_ptr(h_rows, r0)
         _lib.check("mlora_gemm_fwd_fp8", lib.mlora_gemm_fwd_fp8(
-            xq[r0:r1].data_ptr(), xq.stride(0), x_scale[r0:r1].data_ptr(), r1 - r0, K,
+            _row_ptr(xq, r0), xq.stride(0), _row_ptr(x_scale, r0), r1 - r0, K,
             wq.data_ptr(), wq.stride(0), _ptr(w_scale), N,
             _ptr(bias), _DT[bias.dtype] if bias is not None else 0, hr, ldh,
-            ptrs, rk, len(bs), o, i, n, y[r0:r1].data_ptr(), y.stride(0), 0, stream))
+            ptrs, rk, len(bs), o, i, n, _row_ptr(y, r0), y.stride(0), 0, stream))
     return y
 
 
@@ -702,15 +710,14 @@ def f32_shrink(p: torch.Tensor, ops: Sequence[torch.Tensor], op_layout: int, sca
         _require(o.is_contiguous() and o.shape == ((r, K) if op_layout == 0 else (K, r)), "adapter operand shape")
     h = torch.empty((M, width), dtype=torch.float32, device=p.device)
     lib = _lib.load()
-    ptrs, rk, sc = _lib.ptr_array([_ptr(o) for o in ops]), _lib.i32_array(ranks), _lib.f32_array(scales)
+    ptrs, rk, sc = _lib.ptr_array([t.data_ptr() for t in ops]), _lib.i32_array(ranks), _lib.f32_array(scales)
     stream = _stream(p)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
         _lib.check("mlora_f32_shrink", lib.mlora_f32_shrink(
-            p[r0:r1].data_ptr(), p.stride(0), r1 - r0, K, ptrs, op_layout, rk, sc, len(ops), o, i, n,
-            h[r0:r1].data_ptr(), h.stride(0), width, stream))
+            _row_ptr(p, r0), p.stride(0), r1 - r0, K, ptrs, op_layout, rk, sc, len(ops), o, i, n,
+            _row_ptr(h, r0), h.stride(0), width, stream))
     return h
 
 
@@ -729,17 +736,16 @@ def f32_gemm_fwd(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, h:
         _require(b.is_contiguous() and b.shape[0] == N, "lora_b must be contiguous [N, r]")
     y = torch.empty((M, N), dtype=torch.float32, device=x.device)
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(b) for b in bs]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([b.data_ptr() for b in bs]), _lib.i32_array(ranks)
     ldh = h.stride(0) if h is not None else 0
     stream = _stream(x)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
         _lib.check("mlora_f32_gemm_fwd", lib.mlora_f32_gemm_fwd(
-            x[r0:r1].data_ptr(), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N, _ptr(bias),
-            None if h is None else h[r0:r1].data_ptr(), ldh, ptrs, rk, len(bs), o, i, n,
-            y[r0:r1].data_ptr(), y.stride(0), stream))
+            _row_ptr(x, r0), x.stride(0), r1 - r0, K, w.data_ptr(), w.stride(0), N, _ptr(bias),
+            None if h is None else _row_ptr(h, r0), ldh, ptrs, rk, len(bs), o, i, n,
+            _row_ptr(y, r0), y.stride(0), stream))
     return y
 
 
@@ -756,17 +762,16 @@ def f32_gemm_dx(dy: torch.Tensor, w: torch.Tensor, g: torch.Tensor | None, as_: 
         _require(a.is_contiguous(), "lora_a must be contiguous [r, K]")
     dx = torch.empty((M, K), dtype=torch.float32, device=dy.device)
     lib = _lib.load()
-    ptrs, rk = _lib.ptr_array([_ptr(a) for a in as_]), _lib.i32_array(ranks)
+    ptrs, rk = _lib.ptr_array([a.data_ptr() for a in as_]), _lib.i32_array(ranks)
     ldg = g.stride(0) if g is not None else 0
     stream = _stream(dy)
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
+    for r0, r1, o, i, n in routing.call_arrays(_lib.MAX_SEGMENTS):
         if r1 == r0:
             continue
-        o, i, n = _routing_arrays(off, ids)
         _lib.check("mlora_f32_gemm_dx", lib.mlora_f32_gemm_dx(
-            dy[r0:r1].data_ptr(), dy.stride(0), r1 - r0, N, w.data_ptr(), w.stride(0), K,
-            None if g is None else g[r0:r1].data_ptr(), ldg, ptrs, rk, len(as_), o, i, n,
-            dx[r0:r1].data_ptr(), dx.stride(0), stream))
+            _row_ptr(dy, r0), dy.stride(0), r1 - r0, N, w.data_ptr(), w.stride(0), K,
+            None if g is None else _row_ptr(g, r0), ldg, ptrs, rk, len(as_), o, i, n,
+            _row_ptr(dx, r0), dx.stride(0), stream))
     return dx
 
 
@@ -782,14 +787,12 @@ def f32_seg_outer(p: torch.Tensor, h: torch.Tensor, ranks: Sequence[int], routin
     outs: list[torch.Tensor | None] = [None] * len(ranks)
     stream = _stream(p)
     rk = _lib.i32_array(list(ranks))
-    for r0, r1, off, ids in routing.groups(_lib.MAX_SEGMENTS):
-        o, i, n = _routing_arrays(off, ids)
+    for g, (r0, r1, o, i, n) in enumerate(routing.call_arrays(_lib.MAX_SEGMENTS)):
         part = [torch.empty(shape(r), dtype=torch.float32, device=p.device) for r in ranks]
-        ws_bytes = lib.mlora_f32_seg_outer_workspace_bytes(r1 - r0, C, rk, len(ranks), o, i, n)
-        _lib.check("mlora_f32_seg_outer_workspace_bytes", ws_bytes if ws_bytes < 0 else 0)
+        ws_bytes = _outer_workspace("mlora_f32_seg_outer_workspace_bytes", routing, g, C, tuple(ranks))
         ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=p.device) if ws_bytes else None
         _lib.check("mlora_f32_seg_outer_split", lib.mlora_f32_seg_outer_split(
-            p[r0:r1].data_ptr(), p.stride(0), r1 - r0, C, h[r0:r1].data_ptr(), h.stride(0),
+            _row_ptr(p, r0), p.stride(0), r1 - r0, C, _row_ptr(h, r0), h.stride(0),
             _lib.ptr_array([t.data_ptr() for t in part]), out_layout, rk, len(ranks), o, i, n, _ptr(ws), ws_bytes,
             stream))
         outs = [t if acc is None else acc + t for acc, t in zip(outs, part)]

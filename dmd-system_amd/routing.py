@@ -10,6 +10,8 @@ frozen base alone. All routing is host-side integer arithmetic and is exact.
 """
 from __future__ import annotations
 
+import ctypes
+import functools
 from dataclasses import dataclass
 from typing import Iterator, Sequence
 
@@ -86,3 +88,14 @@ class SegmentRouting:
             yield (base, self.seg_offsets[s1],
                    tuple(o - base for o in self.seg_offsets[s0:s1 + 1]),
                    self.adapter_ids[s0:s1])
+
+    def call_arrays(self, max_segments: int) -> list:
+        """``groups`` as the C ABI takes them: (row_start, row_end, int64 offsets, int32 ids, segments) with
+        host arrays (read only, shared by equal routings)."""
+        return _call_arrays(self.seg_offsets, self.adapter_ids, max_segments)
+
+
+@functools.lru_cache(maxsize=256)
+def _call_arrays(seg_offsets: tuple, adapter_ids: tuple, max_segments: int) -> list:
+    return [(r0, r1, (ctypes.c_int64 * len(off))(*off), (ctypes.c_int32 * len(ids))(*ids), len(ids))
+            for r0, r1, off, ids in SegmentRouting(seg_offsets, adapter_ids).groups(max_segments)]
