@@ -44,8 +44,8 @@ struct GemmArgs {
   int32_t accumulate;
   int32_t tiles_m, tiles_n;
   int32_t group_m;  // row tiles per group of the tile order (set by launch_gemm)
-  // >= 0: this launch runs 128x128 quarters of the 256x256 tiles tail_base, tail_base + 1, ... of
-  // the tile order of a tiles_m x tiles_n grid of 256x256 tiles (four workgroups per tile);
+  // >= 0: this launch runs the 128x128 or 64x64 pieces of the 256x256 tiles tail_base, tail_base + 1,
+  // ... of the tile order of a tiles_m x tiles_n grid of 256x256 tiles;
   // -1: one workgroup per tile of its own size (set by launch_gemm)
   int32_t tail_base;
   AdapterTable ext;  // NT: B_a [Ncols, r]; NN: A_a [r, Ncols]
@@ -1348,13 +1348,14 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemm_kernel(con
   const int wm0 = (wave / C::WN) * (C::BM / C::WM);
   const int wn0 = (wave % C::WN) * (C::BN / C::WN);
   int m0, n0;
-  if (C::BM == 128 && C::BN == 128 && args.tail_base >= 0) {
-    // quarter q of the 256x256 tile tail_base + blockIdx.x / 4; a quarter wholly past the
+  if (C::BM < 256 && C::BN < 256 && args.tail_base >= 0) {
+    // piece q of the 256x256 tile tail_base + blockIdx.x / pieces; a piece wholly past the
     // matrix (a narrow last row or column tile) has nothing to compute or store
-    const int q = blockIdx.x % 4;
-    tile_origin<256, 256>(args, args.tail_base + (int)blockIdx.x / 4, m0, n0);
-    m0 += 128 * (q / 2);
-    n0 += 128 * (q % 2);
+    constexpr int PN = 256 / C::BN, PIECES = 256 / C::BM * PN;
+    const int q = blockIdx.x % PIECES;
+    tile_origin<256, 256>(args, args.tail_base + (int)blockIdx.x / PIECES, m0, n0);
+    m0 += C::BM * (q / PN);
+    n0 += C::BN * (q % PN);
     if (m0 >= args.M || n0 >= args.Ncols) return;  // uniform over the workgroup, before any barrier
   } else {
     tile_origin<C::BM, C::BN>(args, blockIdx.x, m0, n0);
@@ -1387,10 +1388,10 @@ using CfgF8128 = GemmCfg<128, 128, 2, 2, false, true>;
 using CfgNN256 = GemmCfg<256, 256, 4, 2, true, false, 128, 2, true, true>;
 using CfgNN128 = GemmCfg<128, 128, 2, 2, true>;
 // NT grids of fewer than 256 tiles of 256x256 (dispatch_nt). Register-buffered steps where a substep
-// is one or two MFMAs: 64x64 tiles of 4 waves (32x32 each; 48 KB, three workgroups per CU) and 128x128
+// is one or two MFMAs: 64x64 tiles of 4 waves (32x32 each; 64 KB, two workgroups per CU) and 128x128
 // tiles of 8 waves (64x32 each; 96 KB), also the quarters of a partly filled last round of 256x256
 // tiles. 128x256 and 256x128 tiles of 8 waves (64x64 each), three stages.
-using CfgNT64 = GemmCfg<64, 64, 2, 2, false, false, 128, 3, false, false, false, true>;
+using CfgNT64 = GemmCfg<64, 64, 2, 2, false, false, 128, 4, false, false, false, true>;
 using CfgNT128 = GemmCfg<128, 128, 2, 4, false, false, 128, 3, false, false, false, true>;
 using CfgNT128x256 = GemmCfg<128, 256, 2, 4, false, false, 128, 3>;
 using CfgNT256x128 = GemmCfg<256, 128, 4, 2, false, false, 128, 3>;
@@ -1421,40 +1422,44 @@ static int launch_gemm(GemmArgs &a, hipStream_t stream, int64_t nblocks = -1) {
   return launch_status();
 }
 
-// The 256x256 tiles from `first` on, as 128x128 quarters of configuration Q.
+// The 256x256 tiles from `first` on, as pieces of configuration Q's tile size.
 template <class Q, bool RESID = false, int STK = 0>
 static int launch_tail(GemmArgs &a, hipStream_t stream, int64_t first) {
-  static_assert(Q::BM == 128 && Q::BN == 128, "quarters of 256x256 tiles");
+  static_assert(Q::BM < 256 && Q::BN < 256 && 256 % Q::BM == 0 && 256 % Q::BN == 0, "pieces of 256x256 tiles");
   a.tiles_m = (a.M + 255) / 256;
   a.tiles_n = (a.Ncols + 255) / 256;
   const int64_t tail = (int64_t)a.tiles_m * a.tiles_n - first;
   a.tail_base = (int32_t)first;
   if (a.group_m <= 0) a.group_m = kGroupM;
-  hipLaunchKernelGGL((gemm_kernel<Q, RESID, STK>), dim3((unsigned)(4 * tail)), dim3(Q::THREADS), 0, stream, a);
+  hipLaunchKernelGGL((gemm_kernel<Q, RESID, STK>), dim3((unsigned)(256 / Q::BM * (256 / Q::BN) * tail)), dim3(Q::THREADS), 0, stream, a);
   return launch_status();
 }
 
 // A grid of 256x256 tiles a little over whole rounds of the 256 CUs (1284 tiles at 27280 x 3072:
 // five rounds and four tiles) would spend a whole tile's time on its last few tiles. Those
-// tiles (at most 64, the last of the tile order) then run in a second launch as 128x128
-// quarters of the 8-wave configuration, one round of at most 256 workgroups: config 3's
-// 27280 x 3072 forward and NN dX took 10% and 7% less time per launch, its step 2.9% less.
-// (The 4-wave two-stage 128x128 tile was no faster than no split. Tails of 104 and 128 tiles,
-// two rounds of quarters, were 2-6% faster per launch in isolation but left config 4's step
-// 0.6% slower.)
-constexpr int64_t kCUs = 256, kMaxTail = 64;
+// tiles (at most 64, the last of the tile order) then run in a second launch as smaller pieces, at
+// most two per CU: 64x64 (NT) up to 32 tiles, else 128x128 quarters of 8 waves. Per launch, tail as
+// 256x256 / quarters / 64x64: 27280 x 3072 x 3072 (4 tiles) 426 / 413 / 400 us, K = 14336 1878 /
+// 1768 / 1705; 11200 x 1536, K = 8960 (8) 340 / 290 / 257; 12000 x 1536 x 1536 (26) 73 / 65 / 61;
+// 13000 x 1536, K = 8960 (50) 360 / 303 / 329. (Tails of 104 and 128 tiles, two rounds of quarters,
+// were 2-6% faster per launch in isolation but left a 73728-row step 0.6% slower.)
+constexpr int64_t kCUs = 256, kMaxTail = 64, kMaxSmallTail = 32;
 
 static int64_t tiles_of(const GemmArgs &a, int64_t bm, int64_t bn) {
   return ((a.M + bm - 1) / bm) * ((a.Ncols + bn - 1) / bn);
 }
 
-// At least 256 tiles of 256x256: whole rounds of them, and a short tail as quarters of Q.
+// At least 256 tiles of 256x256: whole rounds of them, and a short tail as pieces (NT: 64x64 for the
+// shortest; quarters of Q).
 template <class Big, class Q, bool RESID = false, int STK = 0>
 static int launch_rounds(GemmArgs &a, hipStream_t stream) {
   const int64_t big = tiles_of(a, 256, 256), tail = big % kCUs;
   if (tail == 0 || tail > kMaxTail) return launch_gemm<Big, RESID, STK>(a, stream);
   const int st = launch_gemm<Big, RESID, STK>(a, stream, big - tail);
   if (st) return st;
+  if constexpr (!Big::NN) {
+    if (tail <= kMaxSmallTail) return launch_tail<CfgNT64, RESID, STK>(a, stream, big - tail);
+  }
   return launch_tail<Q, RESID, STK>(a, stream, big - tail);
 }
 
