@@ -66,7 +66,9 @@ class _Operands:
         self.batch: dict = {}
 
     def _fast(self, t: torch.Tensor) -> bool:
-        return t.is_cuda and t.dtype in (torch.bfloat16, torch.float32) and t.dim() == 2 and t.stride(1) == 1
+        # (rows that overlap, as of an expanded or a one-row transposed matrix, take the torch ops)
+        return (t.is_cuda and t.dtype in (torch.bfloat16, torch.float32) and t.dim() == 2 and t.stride(1) == 1
+                and t.stride(0) >= t.shape[1])
 
     def _queue(self, t, hi, lo):
         srcs, his, los = self.batch.setdefault(t.dtype, ([], [], []))
