@@ -662,7 +662,7 @@ def main():
     gem_ach = gem["flops"] / gem["time"] / 1e12
     gem_peak = MFMA_FP8_PEAK_TFLOPS if fp8 else MFMA_FP32_PEAK_TFLOPS if f32 else MFMA_BF16_PEAK_TFLOPS
     roofline = {"kernel": ("gemm_kernel NT e4m3 base (fp8 MFMA) + fused dequantise and bf16 LoRA expand"
-                           if fp8 else "f32_linear_kernel (fp32 MFMA base GEMM + fused LoRA expand)" if f32
+                           if fp8 else "f32_gemm_kernel (fp32 MFMA base GEMM + fused LoRA expand)" if f32
                            else "gemm_kernel NT (base GEMM + fused LoRA expand)")
                 + ", over the 6 block linears (median launch of each, cold caches)",
                 "bound": "mfma", "achieved": round(gem_ach, 1), "peak": gem_peak, "unit": "TFLOP/s",
