@@ -66,9 +66,10 @@ class _Operands:
         self.batch: dict = {}
 
     def _fast(self, t: torch.Tensor) -> bool:
-        # (rows that overlap, as of an expanded or a one-row transposed matrix, take the torch ops)
+        # (rows that overlap, as of an expanded or a one-row transposed matrix, and pitches past the kernel's
+        # 32 bits take the torch ops)
         return (t.is_cuda and t.dtype in (torch.bfloat16, torch.float32) and t.dim() == 2 and t.stride(1) == 1
-                and t.stride(0) >= t.shape[1])
+                and t.shape[1] <= t.stride(0) < 2 ** 31)
 
     def _queue(self, t, hi, lo):
         srcs, his, los = self.batch.setdefault(t.dtype, ([], [], []))

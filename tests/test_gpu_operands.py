@@ -43,19 +43,22 @@ def test_prepared_operands_are_the_torch_conversions(pkg, dev, dtype, shapes, pa
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("form", ["one_row", "expanded"])
-def test_adapters_whose_rows_overlap_are_taken(pkg, dev, dtype, form):
-    """A rank-1 lora_a that is a transposed column (pitch 1) and one of equal rows (pitch 0): the call is
-    the one on contiguous copies."""
+@pytest.mark.parametrize("form", ["one_row", "expanded", "far_rows"])
+def test_adapters_of_any_pitch_are_taken(pkg, dev, dtype, form):
+    """A rank-1 lora_a that is a transposed column (pitch 1), one of equal rows (pitch 0) and a rank-1 one
+    with a pitch past 32 bits: the call is the one on contiguous copies."""
     K, N = 96, 64
     g = torch.Generator().manual_seed(3)
 
     def rand(*shape):
         return torch.randn(*shape, generator=g).to(dev)
 
-    a = (rand(K, 1).to(dtype).t() if form == "one_row" else rand(1, K).to(dtype).expand(4, K)).detach()
+    if form == "far_rows":
+        a = rand(1, K).to(dtype).as_strided((1, K), (2 ** 31, 1))
+    else:
+        a = rand(K, 1).to(dtype).t() if form == "one_row" else rand(1, K).to(dtype).expand(4, K)
     r = a.shape[0]
-    assert a.stride(0) < K
+    assert a.stride(0) < K or a.stride(0) >= 2 ** 31
     x, w, b = rand(40, K).bfloat16(), rand(N, K).bfloat16(), rand(N, r).to(dtype)
     routing = pkg.SegmentRouting.from_lengths([40], [0])
     got, want = (pkg.multi_lora_linear(x, w, None, [m], [b], [1.0], routing)
