@@ -162,15 +162,16 @@ shrink_kernel(const ShrinkArgs args) {
   const int32_t o1_off = 8 * o1_c < r ? o1_row * r * 2 + 16 * o1_c : kOOB;
   const bool kmask = K % 64 != 0;
 
-  auto issue = [&](auto st_c, int kc) {
+  auto issue_tile = [&](auto st_c, auto whole_c, int kc) {
+    constexpr bool WHOLE = decltype(whole_c)::value;
     MLORA_LDS char *base = lds + decltype(st_c)::value * C::STAGE_BYTES;
     const int k0 = kc * 64;
-    const bool live = kc < nk;
+    const bool live = WHOLE || kc < nk;
 #pragma unroll
     for (int i = 0; i < C::P_DMA; ++i) {
       const int q = wave * C::P_DMA + i;  // 8-row block of the P tile (wave-uniform)
       int32_t off = p_off[q & 1];
-      if (!live || (kmask && k0 + p_kc[q & 1] >= K)) off = kOOB;
+      if (!WHOLE && (!live || (kmask && k0 + p_kc[q & 1] >= K))) off = kOOB;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, base + q * 1024, 16, off, 8 * q * ldp_b + 2 * k0, 0, 0);
     }
 #pragma unroll
@@ -185,18 +186,32 @@ shrink_kernel(const ShrinkArgs args) {
       if constexpr (OPL == 0) {
         const int j = 8 * q + (lane >> 3);
         int32_t off = j < r ? p_off[q & 1] - (lane >> 3) * ldp_b + j * K * 2 : kOOB;
-        if (!live || dummy || (kmask && k0 + p_kc[q & 1] >= K)) off = kOOB;
+        if (dummy || (!WHOLE && (!live || (kmask && k0 + p_kc[q & 1] >= K)))) off = kOOB;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst, 16, off, 2 * k0, 0, 0);
       } else {
         const int krow = q * (1024 / C::OPROW_B) + o1_row;  // k row within the tile
         int32_t off = o1_off;
-        if (!live || dummy || k0 + krow >= K) off = kOOB;
+        if (dummy || (!WHOLE && (!live || k0 + krow >= K))) off = kOOB;
         // (the scalar offset goes through a variable: written inline in the builtin call,
         // this expression made the host compilation pass drop the kernel instantiation)
         const int32_t soff = (k0 + q * (1024 / C::OPROW_B)) * r * 2;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst, 16, off, soff, 0, 0);
       }
     }
+  };
+  // Whole k-tiles are loaded without masks, decided once per step: deciding per load took scalar
+  // branches for each of a wave's loads, which is what bounded the steps of a grid that leaves HBM
+  // idle. Cold launches of 512 rows: K = 8960, rank 16 51.0 -> 35.7 us, rank 64 82.5 -> 71.4, rank 128
+  // 109 -> 91; K = 1536 11.8 -> 9.3, 18.8 -> 16.9, 24.2 -> 21.3; 65520 rows (HBM-bound) 47.2 -> 47.0 at
+  // rank 64, 63.4 -> 62.6 at 128. Not with more than 4 operand loads per wave (both parts of a rank-128
+  // master, ranks above 128): the second copy of the loads measured 36 -> 236 us and 77 -> 80 there.
+  constexpr bool MASK_FREE = C::OP_DMA <= 4;
+  const int nwhole = K / 64;
+  auto issue = [&](auto st_c, int kc) {
+    if constexpr (MASK_FREE) {
+      if (kc < nwhole) return issue_tile(st_c, std::true_type{}, kc);
+    }
+    issue_tile(st_c, std::false_type{}, kc);
   };
 
   // ---- fragment addresses (stage-relative)
