@@ -619,49 +619,94 @@ __global__ __launch_bounds__(64 * kNormRowsPerBlock) void norm_backward_fused_ke
 }
 
 // The component gradient [batches, 6, width] (zeros in the other four slots) and its sum over the
-// samples, the table gradient [6, width], from the partial sums: one wave per (slot, 8-feature
-// chunk), lane l adding chunks l, l + 64, ... of a sample in order, then a butterfly.
+// samples, the table gradient [6, width], from the partial sums: one wave per (group of samples, slot,
+// 8-feature chunk), its lanes over a sample's chunks, then a butterfly. With several groups, every group
+// leaves its samples' sum as a row of table_partial, and a second launch adds the rows as the chunks of
+// one sample: a fixed order either way.
+//   FEW (at most 8 chunks per sample): lane l takes feature l % 8 of chunk l / 8, the loads of four samples
+//   in flight together, three butterfly steps of one value;
+//   else lane l takes features 4·(l % 2) .. + 3 of the chunks l / 2, l / 2 + 32, ... of two samples.
+// Latency bounds it, so the groups run in parallel: one wave walking every sample took 1 us for each
+// (the whole backward of 512 samples of 8 tokens x 1536, float32 stream: 516 us, in groups of four 70;
+// 4096 samples of 16 tokens 4670 and 420; up to four samples are one group: 220 us at two of 32760).
 struct NormCompFinishArgs {
-  const float *partial;
+  const float *partial;  // [batches, n_chunks, 2, width]
   void *d_comp, *d_table;  // either may be null
-  int32_t batches, width, n_chunks, si, hi, comp_f32, table_f32;
+  float *table_partial;    // [groups, 2, width]; null: the only group writes d_table
+  int32_t batches, per_group, width, n_chunks, si, hi, comp_f32, table_f32;
 };
 
+// Samples per group: four, or what leaves 256 groups.
+static int finish_group(int64_t batches) { return batches <= 1024 ? 4 : (int)((batches + 255) / 256); }
+
+static int64_t finish_groups(int64_t batches) {
+  const int per = finish_group(batches);
+  return (batches + per - 1) / per;
+}
+
+template <bool FEW>
 __global__ __launch_bounds__(64 * kNormRowsPerBlock) void norm_component_finish_kernel(const NormCompFinishArgs a) {
+  constexpr int V = FEW ? 1 : 4, U = FEW ? 4 : 2;        // features per lane; samples at once
+  constexpr int LPC = 8 / V, CPW = 64 / LPC;             // lanes per chunk; chunks of one load
   const int lane = threadIdx.x & 63, nchunks = a.width / 8;
   const int wv = blockIdx.x * kNormRowsPerBlock + wave_id();
-  if (wv >= 6 * nchunks) return;
-  const int slot = wv / nchunks, c = wv % nchunks;
+  const int group = wv / (6 * nchunks), slot = wv / nchunks % 6, c = wv % nchunks;
+  const int b0 = group * a.per_group, b1 = min(b0 + a.per_group, a.batches);
+  if (b0 >= a.batches) return;
   const bool live = slot == a.si || slot == a.hi;
   const int64_t per = 2 * (int64_t)a.width;
-  float table = 0.f;  // lane i < 8: feature 8c + i
-  auto store = [&](void *base, bool f32, int64_t e, float v) {
-    if (f32) static_cast<float *>(base)[e] = v;
-    else static_cast<uint16_t *>(base)[e] = f32_to_bf16_rne(v);
+  const int tc0 = lane / LPC, e0 = 8 * c + V * (lane % LPC);
+  const MLORA_GLOBAL float *base = gp(a.partial) + tc0 * per + (slot == a.si ? 0 : a.width) + e0;
+  auto store = [&](void *out, bool f32, int64_t e, float v) {
+    if (f32) static_cast<float *>(out)[e] = v;
+    else static_cast<uint16_t *>(out)[e] = f32_to_bf16_rne(v);
   };
-  for (int b = 0; b < a.batches; ++b) {
-    float mine = 0.f;
+  float table[V] = {};
+  for (int b = b0; b < b1; b += U) {
+    float acc[U][V] = {};
     if (live) {
-      const float *p = a.partial + (int64_t)b * a.n_chunks * per + (slot == a.si ? 0 : a.width) + 8 * c;
-      float acc[8];
+      if constexpr (FEW) {
+        if (tc0 < a.n_chunks) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-      for (int tc = lane; tc < a.n_chunks; tc += 64) {
-        float v[8];
-        load8(p + (int64_t)tc * per, true, 0, v);
+          for (int u = 0; u < U; ++u) acc[u][0] = base[(int64_t)min(b + u, b1 - 1) * a.n_chunks * per];
+        }
+      } else {
+        const MLORA_GLOBAL float *p = base + (int64_t)b * a.n_chunks * per;
+        const int64_t next = b + 1 < b1 ? a.n_chunks * per : 0;  // (a lone last sample is read twice)
+#pragma unroll 4
+        for (int tc = tc0; tc < a.n_chunks; tc += CPW, p += CPW * per) {
+          const f32x4 v0 = *(const MLORA_GLOBAL f32x4 *)p, v1 = *(const MLORA_GLOBAL f32x4 *)(p + next);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += v[i];
+          for (int i = 0; i < V; ++i) acc[0][i] += v0[i], acc[1][i] += v1[i];
+        }
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float v = wave_sum(acc[i]);
-        mine = lane == i ? v : mine;
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+          for (int m = LPC; m <= 32; m *= 2) acc[u][i] += __shfl_xor(acc[u][i], m);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (b + u >= b1) break;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        table[i] += acc[u][i];
+        if (lane < LPC && a.d_comp != nullptr)
+          store(a.d_comp, a.comp_f32, ((int64_t)(b + u) * 6 + slot) * a.width + e0 + i, acc[u][i]);
       }
     }
-    table += mine;
-    if (lane < 8 && a.d_comp != nullptr) store(a.d_comp, a.comp_f32, ((int64_t)b * 6 + slot) * a.width + 8 * c + lane, mine);
   }
-  if (lane < 8 && a.d_table != nullptr) store(a.d_table, a.table_f32, (int64_t)slot * a.width + 8 * c + lane, table);
+  if (lane >= LPC) return;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    if (a.table_partial != nullptr) {
+      if (live) a.table_partial[group * per + (slot == a.si ? 0 : a.width) + e0 + i] = table[i];
+    } else if (a.d_table != nullptr) {
+      store(a.d_table, a.table_f32, (int64_t)slot * a.width + e0 + i, table[i]);
+    }
+  }
 }
 
 // Tokens per workgroup: the fewest (a power of two, 8 to 128) that leave at most 512 workgroups, the
@@ -834,8 +879,8 @@ extern "C" int64_t mlora_modulated_norm_backward_fused_workspace_bytes(int64_t b
   if (batches < 0 || tokens < 0 || width < 0) return MLORA_ERR_INVALID;
   if (batches == 0 || tokens == 0) return 0;
   if (tokens > INT32_MAX / batches) return MLORA_ERR_LIMIT;
-  const int64_t chunk = fused_chunk(batches, tokens);
-  return batches * ((tokens + chunk - 1) / chunk) * 2 * width * (int64_t)sizeof(float);
+  const int64_t chunk = fused_chunk(batches, tokens), groups = finish_groups(batches);
+  return (batches * ((tokens + chunk - 1) / chunk) + (groups > 1 ? groups : 0)) * 2 * width * (int64_t)sizeof(float);
 }
 
 extern "C" int mlora_modulated_norm_backward_fused(const void *x, int x_dtype, int64_t x_sb, int64_t x_st,
@@ -895,9 +940,19 @@ extern "C" int mlora_modulated_norm_backward_fused(const void *x, int x_dtype, i
   else launch(integral_constant<int, 3>{}, integral_constant<int, 4>{});
   int st = launch_status();
   if (st || (d_comp == nullptr && d_table == nullptr)) return st;
-  const NormCompFinishArgs f{a.partial, d_comp, d_table, (int32_t)batches, (int32_t)width, a.n_chunks, scale_index,
-                             shift_index, d_comp_dtype == MLORA_F32, d_table_dtype == MLORA_F32};
-  const int waves = 6 * (int)(width / 8);
-  hipLaunchKernelGGL(norm_component_finish_kernel, dim3((waves + kNormRowsPerBlock - 1) / kNormRowsPerBlock), block, 0, s, f);
-  return launch_status();
+  const int64_t groups = finish_groups(batches);
+  float *rows_of_groups = groups > 1 && d_table != nullptr ? a.partial + batches * a.n_chunks * 2 * width : nullptr;
+  auto finish = [&](const NormCompFinishArgs &f, int64_t n) {
+    const int64_t waves = n * 6 * (width / 8);
+    const dim3 grid((unsigned)((waves + kNormRowsPerBlock - 1) / kNormRowsPerBlock));
+    if (f.n_chunks <= 8) hipLaunchKernelGGL(norm_component_finish_kernel<true>, grid, block, 0, s, f);
+    else hipLaunchKernelGGL(norm_component_finish_kernel<false>, grid, block, 0, s, f);
+    return launch_status();
+  };
+  const bool cf = d_comp_dtype == MLORA_F32, tf = d_table_dtype == MLORA_F32;
+  st = finish({a.partial, d_comp, d_table, rows_of_groups, (int32_t)batches, finish_group(batches), (int32_t)width,
+               a.n_chunks, scale_index, shift_index, cf, tf}, groups);
+  if (st || rows_of_groups == nullptr) return st;
+  return finish({rows_of_groups, nullptr, d_table, nullptr, 1, 1, (int32_t)width, (int32_t)groups, scale_index, shift_index,
+                 cf, tf}, 1);
 }
