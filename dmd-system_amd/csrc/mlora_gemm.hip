@@ -813,7 +813,7 @@ __device__ __forceinline__ void phase_barrier() {
 // the end of each of its read phases (vmcnt(8)): a load has three phases to land.
 //
 // The last step drains every wave's loads before the last barrier; after it X stages its rows
-// while Y still multiplies, so the epilogue (store_staged) needs no workgroup barrier.
+// while Y still multiplies, so the epilogue (stage_tile, store_rows) needs no workgroup barrier.
 //
 // The k-tiles are contract_tile's sequence (the main contraction, then the LoRA tiles), walked
 // by both sides; X's P loads trail its walk by one k-tile. Each accumulator takes its MFMAs in
@@ -1144,14 +1144,13 @@ struct EpiVectors {
   }
 };
 
-// Staged store: the rounded tile goes to LDS (whose operand stages must be free), row-major with
-// 16-byte chunk q of row r at slot q ^ (r % CH), and leaves in 16-byte stores that cover whole
-// rows. Lane l writes its 8 bytes of (i, j, g) to row wm0 + 32i + l%32, slot
+// Staged store: the rounded tile goes to LDS (stage_tile; the operand stages must be free), row-major
+// with 16-byte chunk q of row r at slot q ^ (r % CH), and leaves in 16-byte stores that cover whole
+// rows (store_rows). Lane l writes its 8 bytes of (i, j, g) to row wm0 + 32i + l%32, slot
 // (wn0/8 + 4j + g) ^ (l%32 % CH): one XOR per (j, g), the row part an immediate offset.
-template <class C, int BK, bool RESID>
-__device__ __forceinline__ void store_staged(const f32x16 (&acc)[C::TM][C::TN], const GemmArgs &args,
-                                             MLORA_LDS char *lds, int m0, int n0, int wm0, int wn0, int lane,
-                                             uint16_t *Ybase, int ncol0) {
+template <class C, int BK>
+__device__ __forceinline__ void stage_tile(const f32x16 (&acc)[C::TM][C::TN], const GemmArgs &args,
+                                           MLORA_LDS char *lds, int m0, int n0, int wm0, int wn0, int lane) {
   constexpr int ROWB = C::BN * 2;  // bytes per staged row
   constexpr int CH = C::BN / 8;    // 16-byte chunks per staged row
   static_assert(C::LDS_BYTES >= C::BM * ROWB, "the staged output tile fits the operand stages");
@@ -1192,9 +1191,16 @@ __device__ __forceinline__ void store_staged(const f32x16 (&acc)[C::TM][C::TN], 
       }
     }
   }
-  // Each wave stores the block it staged itself: (BM / WM) rows of (BN / WN) columns, in 1 KB
-  // instructions of whole 16-byte chunks. It reads only its own LDS writes, so a wave-level
-  // ordering suffices (no workgroup barrier).
+}
+
+// Each wave stores the block it staged itself: (BM / WM) rows of (BN / WN) columns, in 1 KB
+// instructions of whole 16-byte chunks. It reads only its own LDS writes, so a wave-level
+// ordering suffices (no workgroup barrier).
+template <class C, bool RESID>
+__device__ __forceinline__ void store_rows(const GemmArgs &args, MLORA_LDS char *lds, int m0, int n0, int wm0, int wn0,
+                                           int lane, uint16_t *Ybase, int ncol0) {
+  constexpr int ROWB = C::BN * 2, CH = C::BN / 8;
+  const int w8 = wn0 >> 3;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1217,64 +1223,77 @@ __device__ __forceinline__ void store_staged(const f32x16 (&acc)[C::TM][C::TN], 
       buf_store16_nt(ry, offset_of(r), staged(r));
     }
   } else {
-    // Gated residual: x (8 columns of a row, 16 or 32 bytes) and gate come in before any store of a
-    // batch of RBATCH rows, so that a wave has RBATCH rows of loads in flight (one row at a time,
-    // load, add, store: 390 us a launch at 65520 x 1536 x 1536 on the float32 stream, 378 on a bf16
-    // one; in batches 381 and 347; without the residual 290). The output may be x itself: a
-    // lane reads exactly the elements it then writes. When the tile lies
-    // in one gate row (a sample's tokens), its 8 gate values are loaded once.
-    constexpr int RBATCH = (WROWS / RPI) % 8 == 0 ? 8 : (WROWS / RPI) % 4 == 0 ? 4 : 1;
-    const bool one_gate = m0 / args.gate_rows == (m0 + rows_here - 1) / args.gate_rows;  // uniform
-    auto load8f = [&](const float *p, float (&v)[8]) {
-      const f32x4 a = *(const MLORA_GLOBAL f32x4 *)p, b = *(const MLORA_GLOBAL f32x4 *)(p + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = a[e], v[e + 4] = b[e];
-    };
-    float g1[8];
-    if (one_gate && n < args.Ncols) load8f(args.gate + (int64_t)(m0 / args.gate_rows) * args.ldgate + n, g1);
-#pragma unroll
-    for (int i0 = 0; i0 < WROWS / RPI; i0 += RBATCH) {
-      float xs[RBATCH][8];
-#pragma unroll
-      for (int u = 0; u < RBATCH; ++u) {
-        const int r = row_of(i0 + u);
-        const int64_t m = m0 + r;
-        if (offset_of(r) == kOOB) continue;
-        if (args.res_f32) {
-          load8f((const float *)args.res + m * args.ldres + n, xs[u]);
-        } else {
-          const u32x4 xv = *(const MLORA_GLOBAL u32x4 *)((const uint16_t *)args.res + m * args.ldres + n);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xs[u][e] = bf16_to_f32((uint16_t)(e % 2 ? xv[e / 2] >> 16 : xv[e / 2] & 0xffff));
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < RBATCH; ++u) {
-        const int r = row_of(i0 + u);
-        const int64_t m = m0 + r;
-        const int32_t off = offset_of(r);
-        if (off == kOOB) continue;
+    // Gated residual: x (8 columns of a row, 16 or 32 bytes) and gate of the next batch of rows are loaded
+    // before this batch's stores, so that no load waits for a store. The output may be x itself: a lane
+    // reads exactly the elements it then writes. A tile that lies in one gate row (a sample's tokens)
+    // loads its 8 gate values once, one with several (a gate per token, samples that end inside the
+    // tile) each row's. Lanes past the matrix load its last row or first columns and store nothing: no
+    // branch parts the loads. A launch at 65520 x 1536 x 1536, float32 / bf16 stream: one gate per sample
+    // 383 / 306 us, one per token 459 / 372 (row after row, each load, add, store: 408 / 394 and 464 /
+    // 419; batches of loads between the stores, a token's gate at its use: 394 / 364 and 475 / 440;
+    // without the residual 290).
+    constexpr int NR = WROWS / RPI, RB = NR % 4 == 0 ? 4 : NR % 2 == 0 ? 2 : 1;
+    const int nc = n < args.Ncols ? n : 0;
+    auto rows = [&](auto one_c, auto f32_c) {
+      constexpr bool ONE = decltype(one_c)::value, F = decltype(f32_c)::value;
+      struct Row {
+        u32x4 x[F ? 2 : 1];
+        f32x4 g[2];
+      };
+      auto gate = [&](int m, Row &o) {
+        const float *p = args.gate + (int64_t)((uint32_t)m / (uint32_t)args.gate_rows) * args.ldgate + nc;
+        o.g[0] = *(const MLORA_GLOBAL f32x4 *)p, o.g[1] = *(const MLORA_GLOBAL f32x4 *)(p + 4);
+      };
+      auto load = [&](int it, Row &o) {
+        const int m = m0 + min(row_of(it), rows_here - 1);
+        const MLORA_GLOBAL char *p = (const MLORA_GLOBAL char *)args.res + ((int64_t)m * args.ldres + nc) * (F ? 4 : 2);
+        o.x[0] = *(const MLORA_GLOBAL u32x4 *)p;
+        if constexpr (F) o.x[1] = *(const MLORA_GLOBAL u32x4 *)(p + 16);
+        if constexpr (!ONE) gate(m, o);
+      };
+      Row one;
+      if constexpr (ONE) gate(m0, one);
+      auto put = [&](int it, const Row &b) {
+        const int r = row_of(it);
         const u32x4 d = staged(r);  // 8 values of bf16(Y)
-        float g[8], o[8];
-        if (one_gate) {
+        float o[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) g[e] = g1[e];
-        } else {
-          load8f(args.gate + (m / args.gate_rows) * args.ldgate + n, g);
+        for (int e = 0; e < 8; ++e) {
+          const float x = F ? __uint_as_float(b.x[e / 4 * F][e % 4])
+                            : bf16_to_f32((uint16_t)(e % 2 ? b.x[0][e / 2] >> 16 : b.x[0][e / 2] & 0xffff));
+          o[e] = gated_add(x, bf16_to_f32((uint16_t)(e % 2 ? d[e / 2] >> 16 : d[e / 2] & 0xffff)),
+                           (ONE ? one : b).g[e / 4][e % 4]);
         }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          o[e] = gated_add(xs[u][e], bf16_to_f32((uint16_t)(e % 2 ? d[e / 2] >> 16 : d[e / 2] & 0xffff)), g[e]);
-        if (args.res_f32) {
+        if constexpr (F) {
           // float32 stream: no bf16 rounding of the sum; 32 bytes per lane
-          MLORA_GLOBAL f32x4 *op = (MLORA_GLOBAL f32x4 *)(args.Yf + m * args.ldy + n);
+          if (offset_of(r) == kOOB) return;
+          MLORA_GLOBAL f32x4 *op = (MLORA_GLOBAL f32x4 *)(args.Yf + (int64_t)(m0 + r) * args.ldy + n);
           op[0] = f32x4{o[0], o[1], o[2], o[3]};
           op[1] = f32x4{o[4], o[5], o[6], o[7]};
         } else {
-          buf_store16_nt(ry, off, u32x4{pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3]), pack2_bf16(o[4], o[5]),
-                                        pack2_bf16(o[6], o[7])});
+          buf_store16_nt(ry, offset_of(r), u32x4{pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3]), pack2_bf16(o[4], o[5]),
+                                                 pack2_bf16(o[6], o[7])});
         }
+      };
+      Row b[2][RB];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) load(u, b[0][u]);
+#pragma unroll
+      for (int i0 = 0; i0 < NR; i0 += RB) {
+        const int cur = i0 / RB % 2;
+        if (i0 + RB < NR) {
+#pragma unroll
+          for (int u = 0; u < RB; ++u) load(i0 + RB + u, b[cur ^ 1][u]);
+        }
+#pragma unroll
+        for (int u = 0; u < RB; ++u) put(i0 + u, b[cur][u]);
       }
+    };
+    const bool one = m0 / args.gate_rows == (m0 + rows_here - 1) / args.gate_rows;  // uniform, as is res_f32
+    if (args.res_f32) {
+      if (one) rows(std::true_type{}, std::true_type{}); else rows(std::false_type{}, std::true_type{});
+    } else {
+      if (one) rows(std::true_type{}, std::false_type{}); else rows(std::false_type{}, std::false_type{});
     }
   }
 }
@@ -1329,9 +1348,15 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[C::TM][C::TN], co
     else store_direct<C, 0>(acc, args, m0, n0, wm0, wn0, lane, Ybase, ncol0);
     return;
   }
-  if (args.bias_dtype == MLORA_BF16) store_staged<C, 1, RESID>(acc, args, lds, m0, n0, wm0, wn0, lane, Ybase, ncol0);
-  else if (args.bias_dtype == MLORA_F32) store_staged<C, 2, RESID>(acc, args, lds, m0, n0, wm0, wn0, lane, Ybase, ncol0);
-  else store_staged<C, 0, RESID>(acc, args, lds, m0, n0, wm0, wn0, lane, Ybase, ncol0);
+  auto put = [&](auto bk) {
+    stage_tile<C, decltype(bk)::value>(acc, args, lds, m0, n0, wm0, wn0, lane);
+    if constexpr (!RESID) store_rows<C, false>(args, lds, m0, n0, wm0, wn0, lane, Ybase, ncol0);
+  };
+  if (args.bias_dtype == MLORA_BF16) put(std::integral_constant<int, 1>{});
+  else if (args.bias_dtype == MLORA_F32) put(std::integral_constant<int, 2>{});
+  else put(std::integral_constant<int, 0>{});
+  // (once, not per bias kind: three copies of the residual's rows made the 256x256 kernel spill)
+  if constexpr (RESID) store_rows<C, true>(args, lds, m0, n0, wm0, wn0, lane, Ybase, ncol0);
 }
 
 // One workgroup per output tile. RESID: the stored value is the block's gated

@@ -152,3 +152,37 @@ def test_fused_gated_residual_float32_stream(pkg, dev, M, K, N, samples):
     assert torch.equal(xs[0].grad, xs[1].grad)
     for p0, p1 in zip(Ag[0] + Bg[0], Ag[1] + Bg[1]):
         assert torch.equal(p0.grad, p1.grad)
+
+
+@pytest.mark.parametrize("stream", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N", [
+    (70, 72),       # 64x64 tiles, cut in both directions
+    (2300, 1544),   # 128x128
+    (4300, 1544),   # 256x128
+    (4600, 1536),   # 128x256
+    (6400, 1544),   # one partly filled round of 256x256
+    (10000, 1544),  # a round of 256x256 and a tail as 64x64 pieces
+    (13000, 1536),  # ... and as 128x128 quarters
+])
+def test_gated_rows_in_every_tile(pkg, dev, M, N, stream):
+    """Every tile's epilogue with one gate row for all rows, one per row, and gate rows that end inside
+    the tiles, on a residual whose rows are apart (not-a-numbers between them), out of place and in
+    place: bit-exact against the unfused product and two float32 operations. Each bias kind once."""
+    K, k = 96, pkg.kernels
+    cut = M // 3
+    routing = pkg.SegmentRouting.from_lengths((cut, 1, M - cut - 1), (0, -1, 1))
+    x, w, b, _, Bs, _, _ = _case(dev, M, K, N, (32, 16), (M,), (0,), seed=M + N, samples=1)
+    g = torch.Generator(device=dev).manual_seed(M)
+    h = (torch.randn(M, 32, generator=g, device=dev) * 0.3).bfloat16()
+    wide = torch.full((M, N + 8), float("nan"), device=dev, dtype=stream)
+    wide[:, :N] = torch.randn(M, N, generator=g, device=dev)
+    res = wide[:, :N]
+    for per, bias in ((M, None), (1, b), (10, b.float())):
+        gate = torch.randn(M // per, N, generator=g, device=dev)
+        y = k.gemm_fwd(x, w, bias, h, Bs, routing)
+        want = (res.float() + y.float() * gate.repeat_interleave(per, dim=0)).to(stream)
+        got = k.gemm_fwd_gated(x, w, bias, h, Bs, routing, res, gate)
+        assert torch.equal(got, want), per
+        place = wide.clone()
+        k.gemm_fwd_gated(x, w, bias, h, Bs, routing, place[:, :N], gate, out=place[:, :N])
+        assert torch.equal(place[:, :N], want) and place[:, N:].isnan().all(), per
