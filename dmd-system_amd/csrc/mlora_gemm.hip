@@ -1418,6 +1418,11 @@ using CfgNN128 = GemmCfg<128, 128, 2, 2, true>;
 // tiles. 128x256 and 256x128 tiles of 8 waves (64x64 each), three stages.
 using CfgNT64 = GemmCfg<64, 64, 2, 2, false, false, 128, 4, false, false, false, true>;
 using CfgNT128 = GemmCfg<128, 128, 2, 4, false, false, 128, 3, false, false, false, true>;
+// Contractions of few k-tiles: 128x128 tiles whose steps read LDS substep by substep (a register-buffered
+// step reads a whole k-tile ahead, too few of which are left to hide it), of 8 waves (32x64 each,
+// three stages) or of 4 (64x64 each, two workgroups per CU).
+using CfgNT128S = GemmCfg<128, 128, 4, 2, false, false, 128, 3>;
+using CfgNT128D = GemmCfg<128, 128, 2, 2, false>;
 using CfgNT128x256 = GemmCfg<128, 256, 2, 4, false, false, 128, 3>;
 using CfgNT256x128 = GemmCfg<256, 128, 4, 2, false, false, 128, 3>;
 // 128x128 NN tiles of 8 waves (64x32 each) with three stages (two k-tiles in flight), one workgroup
@@ -1508,13 +1513,19 @@ static int launch_rounds(GemmArgs &a, hipStream_t stream) {
 // * up to 128 tiles of 128x128: 64x64 tiles (at most 512, two per CU);
 // * up to 256: 128x128, one per CU;
 // * while 128x256 or 256x128 tiles (whichever are fewer) fit one round: those;
-// * else 256x256, in one partly filled round or (from 256 tiles on) whole rounds and a tail.
+// * else 256x256, in one partly filled round or (from 256 tiles on) whole rounds and a tail;
+// * contractions below 448 (of one stacked linear, where dX has several): CfgNT128S in place of the
+//   128x128 tile and CfgNT128D while two per CU hold the grid. 13000 x 256 x 256: 9.6 and 9.1 us, 20000 x 256
+//   x 256: 11.1 and 10.3, dX of three 256-wide linears at 13000 rows 17.4 and 16.3; even from K = 448 on
+//   (20000 x 256 x 640 16.9, CfgNT128D 17.9).
 template <bool RESID = false, int STK = 0>
 static int dispatch_nt(GemmArgs &a, hipStream_t stream) {
   if (tiles_of(a, 256, 256) >= kCUs) return launch_rounds<CfgNT256, CfgNT128, RESID, STK>(a, stream);
   const int64_t mid = tiles_of(a, 128, 128);
+  const bool few = (STK == 2 ? a.group_cols : a.Kc) < 448;  // k-tiles of one source
   if (mid <= kCUs / 2) return launch_gemm<CfgNT64, RESID, STK>(a, stream);
-  if (mid <= kCUs) return launch_gemm<CfgNT128, RESID, STK>(a, stream);
+  if (mid <= kCUs) return few ? launch_gemm<CfgNT128S, RESID, STK>(a, stream) : launch_gemm<CfgNT128, RESID, STK>(a, stream);
+  if (mid <= 2 * kCUs && few) return launch_gemm<CfgNT128D, RESID, STK>(a, stream);
   const int64_t wide = tiles_of(a, 128, 256), tall = tiles_of(a, 256, 128);
   if (wide <= kCUs && wide <= tall) return launch_gemm<CfgNT128x256, RESID, STK>(a, stream);
   if (tall <= kCUs) return launch_gemm<CfgNT256x128, RESID, STK>(a, stream);

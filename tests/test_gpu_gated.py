@@ -155,20 +155,21 @@ def test_fused_gated_residual_float32_stream(pkg, dev, M, K, N, samples):
 
 
 @pytest.mark.parametrize("stream", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K", [96, 456])  # either side of the tile rule for short contractions
 @pytest.mark.parametrize("M,N", [
     (70, 72),       # 64x64 tiles, cut in both directions
     (2300, 1544),   # 128x128
-    (4300, 1544),   # 256x128
-    (4600, 1536),   # 128x256
+    (4300, 1544),   # 256x128; K = 96: 128x128, two per CU
+    (4600, 1536),   # 128x256; the same
     (6400, 1544),   # one partly filled round of 256x256
     (10000, 1544),  # a round of 256x256 and a tail as 64x64 pieces
     (13000, 1536),  # ... and as 128x128 quarters
 ])
-def test_gated_rows_in_every_tile(pkg, dev, M, N, stream):
+def test_gated_rows_in_every_tile(pkg, dev, M, N, K, stream):
     """Every tile's epilogue with one gate row for all rows, one per row, and gate rows that end inside
     the tiles, on a residual whose rows are apart (not-a-numbers between them), out of place and in
     place: bit-exact against the unfused product and two float32 operations. Each bias kind once."""
-    K, k = 96, pkg.kernels
+    k = pkg.kernels
     cut = M // 3
     routing = pkg.SegmentRouting.from_lengths((cut, 1, M - cut - 1), (0, -1, 1))
     x, w, b, _, Bs, _, _ = _case(dev, M, K, N, (32, 16), (M,), (0,), seed=M + N, samples=1)
