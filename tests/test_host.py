@@ -207,3 +207,18 @@ def test_make_linear_is_seeded(pkg):
             assert all(torch.equal(p, q) for p, q in zip(u, v))
         else:
             assert torch.equal(u, v)
+
+
+# ---------------------------------------------------------------- inputs
+
+@pytest.mark.parametrize("shape", [(3, 0), (0, 0), (2, 3, 0)])
+def test_inputs_without_features_are_refused(pkg, shape):
+    """An empty last dimension has no row count (torch.reshape's rule), for matrices as for batches."""
+    x, w = torch.zeros(shape, dtype=torch.bfloat16), torch.zeros(8, 0, dtype=torch.bfloat16)
+    routing = pkg.SegmentRouting.single(3, -1)
+    for call in (lambda: pkg.multi_lora_linear(x, w, None, [], [], [], routing),
+                 lambda: pkg.multi_lora_linear_gated(x, w, None, [], [], [], routing, torch.zeros(*shape[:-1], 8), torch.zeros(1, 8)),
+                 lambda: pkg.multi_lora_linear_fp8(x, w.to(torch.float8_e4m3fn), torch.ones(8), None, [], [], [], routing),
+                 lambda: pkg.shared_input_multi_lora(x, [w], [None], [[]], [[]], [], routing)):
+        with pytest.raises(RuntimeError, match="reshape"):
+            call()
