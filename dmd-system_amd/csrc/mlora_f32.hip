@@ -40,6 +40,9 @@
 
 namespace mlora {
 
+// Pitch (floats) below which direct-to-LDS loads address a whole tile with 31-bit byte offsets.
+constexpr int64_t kDirectLd = (int64_t)1 << 21;
+
 // One contraction source. K-contiguous P: rows [p_lo, p_hi) are valid; natural operands:
 // columns [0, p_hi) / [0, q_hi). klen contraction elements.
 struct F32Src {
@@ -68,6 +71,10 @@ struct F32Cfg {
   static constexpr int LDS_BYTES = RING_BYTES > RED_BYTES ? RING_BYTES : RED_BYTES;
   static_assert(LDS_BYTES <= 163840, "the ring fits the LDS");
   static_assert((STAGES - 2) * LPW < 64, "vmcnt field");
+  // The bytes from a tile's first row (or contraction index) to the end of its last: the widest, 256
+  // rows of a shrink's operand above rank 128, ends 4080 bytes before kOOB.
+  static constexpr int64_t ROWS = BM > BN ? (BM > BK ? BM : BK) : (BN > BK ? BN : BK);
+  static_assert(ROWS * 4 * (kDirectLd - 4) < kOOB, "offsets stay in range at any pitch taken");
   static constexpr int WG_PER_CU = 163840 / LDS_BYTES;
   static constexpr int WAVES_PER_SIMD = NW * WG_PER_CU / 4 > 4 ? 4 : (NW * WG_PER_CU + 3) / 4;
 };
@@ -644,9 +651,9 @@ static int check_f32_matrix(const void *p, int64_t ld, int64_t rows, int64_t col
 }
 
 // 16-byte direct-to-LDS loads can read the matrix: whole chunks of 4, and the byte offsets of a
-// tile (at most 128 rows or contraction indices) stay 31-bit.
+// tile (up to 256 rows, F32Cfg) stay below the out-of-range one.
 static bool direct_ok(const void *p, int64_t ld, int64_t cols) {
-  return aligned16(p) && ld % 4 == 0 && cols % 4 == 0 && ld < ((int64_t)1 << 21);
+  return aligned16(p) && ld % 4 == 0 && cols % 4 == 0 && ld < kDirectLd;
 }
 
 // Adapter operands for the fp32 kernels: any rank in [0, kMaxRank] (no padding). direct: cleared
