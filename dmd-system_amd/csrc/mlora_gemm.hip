@@ -538,8 +538,6 @@ __device__ __forceinline__ void contract_tile(f32x16 (&acc)[C::TM][C::TN], const
               0, args.M, args.Kc, esz0};
   int bk = C::KB / src.esz;  // contraction elements per k-tile of the current source
   int ntile = (src.klim + bk - 1) / bk;
-  // e4m3: the main contraction is padded to a multiple of S k-tiles (zero
-  // chunks) so the bf16 LoRA k-tiles start at stage 0
   const int n_main = ntile;  // e4m3 k-tiles (F8), before the first LoRA tile
   if (ntile == 0) {
     first_seg();
