@@ -350,6 +350,95 @@ def test_modulated_norm_backward_rejects_bad_arguments(lib, pkg):
     assert comp(reduce=0, sb=4 * 6 * 64, st=6 * 64, out=0x7004) == L.ERR_UNSUPPORTED
 
 
+def test_fused_norm_backward_rejects_bad_arguments(lib, pkg):
+    L = pkg._lib
+    need = lib.mlora_modulated_norm_backward_fused_workspace_bytes
+
+    def bwd(x=0x10000, g=0x20000, sc=0x30000, srow=0x40000, dx=0x50000, dcomp=0x60000, dtable=0x70000, ws=0x80000,
+            wsb=None, eps=1e-6, W=64, T=4, B=1, dt=0, tdt=0, cdt=0, si=1, hi=0, dxst=None, dxsb=None, scsb=6 * 64):
+        dxst = W if dxst is None else dxst
+        dxsb = T * dxst if dxsb is None else dxsb
+        wsb = need(B, T, W) if wsb is None else wsb
+        return lib.mlora_modulated_norm_backward_fused(x, dt, T * W, W, g, 1, T * W, W, srow, tdt, sc, 0, scsb, dx, dxsb, dxst,
+                                                       eps, si, hi, dcomp, cdt, dtable, cdt, ws, wsb, B, T, W, None)
+
+    assert need(1, 4, 64) == 2 * 64 * 4                 # one chunk of tokens, one group of samples
+    assert need(2, 20, 64) == 2 * 3 * 2 * 64 * 4        # chunks of 8 tokens
+    assert need(5, 4, 64) == (5 + 2) * 2 * 64 * 4       # the second group's and the first's table rows
+    assert need(2000, 4, 64) == (2000 + 250) * 2 * 64 * 4
+    assert need(0, 4, 64) == need(4, 0, 64) == need(4, 4, 0) == 0
+    assert need(-1, 4, 64) == need(1, -4, 64) == need(1, 4, -64) == L.ERR_INVALID
+    assert need(2 ** 20, 2 ** 20, 64) == L.ERR_LIMIT
+    assert bwd(W=5128) == bwd(W=12) == L.ERR_UNSUPPORTED
+    assert bwd(dt=2) == bwd(tdt=2) == bwd(cdt=2) == L.ERR_UNSUPPORTED
+    assert bwd(eps=0.0) == bwd(eps=float("nan")) == bwd(eps=float("inf")) == L.ERR_INVALID
+    assert bwd(si=6) == bwd(hi=-1) == bwd(si=2, hi=2) == L.ERR_INVALID
+    assert bwd(x=None) == bwd(g=None) == bwd(sc=None) == bwd(dx=None) == L.ERR_INVALID
+    assert bwd(g=0x20004) == bwd(srow=0x40008) == bwd(dx=0x50008) == bwd(scsb=6 * 64 + 4) == L.ERR_UNSUPPORTED
+    assert bwd(dxst=32) == bwd(B=2, dxsb=3 * 64) == L.ERR_INVALID  # rows or samples of dx overlap
+    assert bwd(ws=None) == bwd(wsb=need(1, 4, 64) - 4) == L.ERR_WORKSPACE
+    assert bwd(B=5, wsb=need(5, 4, 64) - 4) == L.ERR_WORKSPACE
+    assert bwd(ws=0x80004) == L.ERR_UNSUPPORTED
+    assert bwd(B=-1) == bwd(T=-1, wsb=0) == L.ERR_INVALID
+    assert bwd(B=2 ** 20, T=2 ** 20, wsb=0) == L.ERR_LIMIT
+    assert bwd(B=0) == bwd(T=0, ws=None) == bwd(W=0) == L.OK
+
+
+def test_prepare_operands_rejects_bad_arguments(lib, pkg):
+    L = pkg._lib
+
+    def prep(src=0x1000, dt=0, sld=64, r=8, c=64, pr=8, pc=64, hi=0x2000, lo=0x3000, old=64, t=0x4000, tld=8, n=1, without=None):
+        args = dict(src=L.ptr_array([src]), sld=L.i64_array([sld]), r=L.i64_array([r]), c=L.i64_array([c]), pr=L.i64_array([pr]),
+                    pc=L.i64_array([pc]), hi=L.ptr_array([hi]), lo=L.ptr_array([lo]), old=L.i64_array([old]), t=L.ptr_array([t]),
+                    tld=L.i64_array([tld]))
+        a = {k: None if k == without else v for k, v in args.items()}
+        return lib.mlora_prepare_operands(a["src"], dt, a["sld"], a["r"], a["c"], a["pr"], a["pc"], a["hi"], a["lo"], a["old"],
+                                          a["t"], a["tld"], n, None)
+
+    assert prep(n=-1) == L.ERR_INVALID
+    assert prep(n=0) == L.OK
+    assert prep(dt=2) == L.ERR_UNSUPPORTED
+    assert prep(src=0) == prep(sld=63) == L.ERR_INVALID            # rows to read, none given or overlapping
+    assert prep(pr=7) == prep(pc=56) == L.ERR_INVALID              # padded below the matrix
+    assert prep(r=-1) == prep(c=-1) == L.ERR_INVALID
+    assert prep(old=63) == prep(tld=7) == L.ERR_INVALID            # output rows overlap
+    assert prep(sld=2 ** 31) == prep(old=2 ** 31) == prep(tld=2 ** 31) == L.ERR_LIMIT
+    assert prep(pr=2 ** 31, tld=2 ** 31) == L.ERR_LIMIT
+    assert prep(hi=0, lo=0, t=0, old=0, tld=0) == L.OK             # nothing asked for
+    assert prep(r=0, c=0, pr=0, pc=0, src=0) == L.OK
+    for name in ("src", "sld", "r", "c", "pr", "pc", "hi", "lo", "old", "t", "tld"):
+        assert prep(without=name) == L.ERR_INVALID                 # every array is required
+
+
+def test_f32_split_reduction_rejects_bad_arguments(lib, pkg):
+    L = pkg._lib
+    off, ids, ranks = L.i64_array([0, 3000]), L.i32_array([0]), L.i32_array([64])
+
+    def need(M=3000, C=1536, rk=ranks, n=1, o=off, i=ids, s=1):
+        return lib.mlora_f32_seg_outer_workspace_bytes(M, C, rk, n, o, i, s)
+
+    def outer(p=0x10000, h=0x20000, ldh=64, outs=(0x30000,), layout=0, ws=0x40000, wsb=None, o=off, rk=ranks):
+        wsb = need() if wsb is None else wsb
+        return lib.mlora_f32_seg_outer_split(p, 1536, 3000, 1536, h, ldh, L.ptr_array(list(outs)), layout, rk, 1, o, ids, 1,
+                                             ws, wsb, None)
+
+    splits, rest = divmod(need(), 4 * 1536 * 64)
+    assert splits == 12 and rest == 0                    # runs of 256 of the 3000 rows
+    assert need(M=200, o=L.i64_array([0, 200])) == 0     # one run: written straight to the output
+    assert need(i=L.i32_array([-1])) == 0                # no rows
+    assert need(rk=L.i32_array([0])) == 0
+    assert need(rk=L.i32_array([-1])) == need(o=L.i64_array([0, 2999])) == need(i=L.i32_array([1])) == L.ERR_INVALID
+    assert need(rk=L.i32_array([L.MAX_RANK + 1])) == need(M=2 ** 31) == need(C=-1) == L.ERR_LIMIT
+    assert need(rk=None) == L.ERR_INVALID
+    assert outer(ws=None) == outer(wsb=need() - 4) == L.ERR_WORKSPACE
+    assert outer(ws=0x40004) == L.ERR_UNSUPPORTED
+    assert outer(layout=2) == outer(outs=(0,)) == outer(outs=(0x30002,)) == L.ERR_INVALID
+    assert outer(p=0) == outer(h=0) == outer(ldh=63) == L.ERR_INVALID
+    assert outer(p=0x10002) == L.ERR_UNSUPPORTED
+    assert outer(o=L.i64_array([0, 2999])) == L.ERR_INVALID
+    assert outer(rk=L.i32_array([0]), ws=None, wsb=0) == L.OK
+
+
 # ---------------------------------------------------------------- host-side sizing, random routings
 
 from hypothesis import given, settings, strategies as st  # noqa: E402
