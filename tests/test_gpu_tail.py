@@ -1,14 +1,14 @@
 """Grids of 256x256 output tiles a little over whole rounds of the 256 CUs.
 
 Such a grid (1284 tiles at 27280 x 3072: five rounds and four tiles) runs its whole rounds as
-256x256 tiles and its last few tiles (at most 64) as 128x128 quarters (8 waves) in a second
-launch. Every output keeps its k order and MFMA sequence in all tile sizes, so the GEMMs must
-give the same bits as calls on row blocks of 1024 rows (fewer than 256 tiles: 128x128 tiles
-throughout), and the fp64 oracle's result within the bf16 tolerance. Covered: the forward
-GEMM with bias and three rank-128 segments (config 3's routing), the NN dX, a tail of 64 tiles
-(5000 x 4096: 256 quarters), one of 104 tiles (27280 x 14336, run as 256x256 tiles), quarters
-wholly past the matrix (a last row tile of 100 rows and a last column tile of 128 columns), the
-stacked forward and dX of three linears that read one input, the gated-residual epilogue on bf16
+256x256 tiles and its last few tiles (at most 64) as smaller pieces in a second launch: 64x64
+(the NT forms, up to 32 tiles) or 128x128 quarters (8 waves). Every output keeps its k order and
+MFMA sequence in all tile sizes, so the GEMMs must give the same bits as calls on row blocks of
+1024 rows (fewer than 256 tiles of 256x256), and the fp64 oracle's result within the bf16
+tolerance. Covered: the forward GEMM with bias and three rank-128 segments (config 3's routing),
+the NN dX, a tail of 64 tiles (5000 x 4096: 256 quarters), one of 104 tiles (27280 x 14336, run as
+256x256 tiles), pieces wholly past the matrix (a last row tile of 100 rows and a last column tile
+of 128 columns), the stacked forward and dX of three linears that read one input, the gated-residual epilogue on bf16
 and float32 streams, and the e4m3 forward (which runs its tail as 256x256 tiles).
 """
 import math
