@@ -716,6 +716,8 @@ static int launch_f32_gemm(F32LinArgs &a, hipStream_t stream) {
 //     LoRA term); 4680 rows: 64x64 187, 128x64 212, 128x128 222;
 //   512 x 1536 x 1536 (192 tiles of 64x64): two wave groups splitting the contraction 36 us, one 38.
 // Before (128x128 tiles, element loads, k-tiles of 16): 1160 us at 9360 rows.
+// Element loads of the same call (one rank off a multiple of 4 sends the base there too): 690 us at 9360
+// rows (direct 390 on that box, the kernels before 1070), 335 at 4680 (209, 560).
 template <bool QN, bool DIRECT>
 static int dispatch_f32_gemm(F32LinArgs &a, hipStream_t stream) {
   const int64_t wide = (((int64_t)a.M + 127) / 128) * (((int64_t)a.Ncols + 63) / 64);
