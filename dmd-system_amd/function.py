@@ -689,9 +689,10 @@ def _autocast_bf16() -> bool:
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
-    """t [..., K] as rows [M, K] (a matrix stays itself: no view node in the graph; one without columns
-    goes through the reshape, which refuses it as it does any other empty last dimension)."""
-    return t if t.dim() == 2 and t.shape[1] else t.reshape(-1, t.shape[-1])
+    """t [..., K] as rows [M, K] (a matrix stays itself: no view node in the graph). One row, or none, goes
+    through the reshape: it counts as contiguous whatever its pitch, which the kernels would be given. So does
+    a matrix without columns, which the reshape refuses as it does any other empty last dimension."""
+    return t if t.dim() == 2 and t.shape[0] > 1 and t.shape[1] else t.reshape(-1, t.shape[-1])
 
 
 def _unrows(y: torch.Tensor, lead) -> torch.Tensor:

@@ -64,3 +64,35 @@ def test_adapters_of_any_pitch_are_taken(pkg, dev, dtype, form):
     got, want = (pkg.multi_lora_linear(x, w, None, [m], [b], [1.0], routing)
                  for m in (a, a.clone(memory_format=torch.contiguous_format)))
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("path", ["bf16", "f32", "fp8", "gated", "shared"])
+def test_one_row_of_a_wider_matrix_is_taken(pkg, dev, path):
+    """A single row x [1, K] counts as contiguous at any pitch; the call is the one on a copy."""
+    K, N, r = 64, 256, 16
+    g = torch.Generator().manual_seed(5)
+    dt = torch.float32 if path == "f32" else torch.bfloat16
+
+    def rand(*shape, dtype=dt):
+        return torch.randn(*shape, generator=g).to(dev, dtype)
+
+    x, res, up = rand(1, K + 1)[:, :K], rand(1, N + 3, dtype=torch.float32)[:, :N], rand(1, N)
+    assert x.stride(0) == K + 1 and x.is_contiguous()
+    w, a, b, gate = rand(N, K), rand(r, K), rand(N, r), rand(1, N, dtype=torch.float32)
+    routing = pkg.SegmentRouting.single(1)
+
+    def call(x, res):
+        ls = [t.clone().requires_grad_(True) for t in (a, b)]
+        leaf = x.detach().requires_grad_(True)
+        if path == "fp8":
+            y = pkg.multi_lora_linear_fp8(leaf, *pkg.kernels.quantize_rows_fp8(w), None, ls[:1], ls[1:], [1.0], routing)
+        elif path == "gated":
+            y = pkg.multi_lora_linear_gated(leaf, w, None, ls[:1], ls[1:], [1.0], routing, res, gate)
+        elif path == "shared":
+            y = sum(pkg.shared_input_multi_lora(leaf, [w, w], [None] * 2, [ls[:1]] * 2, [ls[1:]] * 2, [1.0], routing))
+        else:
+            y = pkg.multi_lora_linear(leaf, w, None, ls[:1], ls[1:], [1.0], routing)
+        return [y.detach(), *torch.autograd.grad(y, [leaf, *ls], up.to(y.dtype))]
+
+    for got, want in zip(call(x, res), call(x.reshape(-1).clone().view(1, K), res.reshape(-1).clone().view(1, N))):
+        assert torch.equal(got, want)
